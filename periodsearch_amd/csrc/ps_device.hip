@@ -139,6 +139,129 @@ bool build_schedule(const std::vector<int> &lc_start, const std::vector<int> &lc
     }
     return true;
 }
+
+// The symmetry orbits of a geometry (ps_orbit.h): for every orbit the representative's normal and
+// harmonics, for every facet its entry (8 * orbit + 2k + (1: -n_k)).  Returns false where the mesh or the
+// coefficient set is not of that kind (a caller may fill ps_geometry itself); every member's normal and
+// harmonics are compared with what the symmetry gives, to a few units of rounding.
+struct Orbits {
+    int L = 0, n = 0;
+    std::vector<double> table;
+    std::vector<unsigned> corr;  // [32 positions][orbit, one more][position][member]: member - symmetric, bfloat16 pairs
+    std::vector<int> pos, coef;
+};
+unsigned bf16_bits(double x) {  // round to nearest even (finite x)
+    const float f = float(x);
+    unsigned u;
+    std::memcpy(&u, &f, 4);
+    return (u + 0x7fff + ((u >> 16) & 1)) >> 16;
+}
+template <int L>
+void orbit_stream(std::vector<int> &l, std::vector<int> &m, std::vector<int> &sn) {
+    constexpr psk::OrbLayout<L> lay{};
+    l.assign(lay.l, lay.l + lay.N);
+    m.assign(lay.m, lay.m + lay.N);
+    sn.assign(lay.sn, lay.sn + lay.N);
+}
+bool build_orbits(const ps_geometry &g, Orbits &ob) {
+    if (g.lmax < 0 || g.lmax > psk::kOrbMaxL || g.mmax > g.lmax || g.nfac % 8 != 0 || g.nfac > kMaxFac) return false;
+    // the coefficients in the order of the tables: m, then l >= m, cos and (m > 0) sin
+    std::map<std::tuple<int, int, int>, int> index;
+    int q = 0, k = 0;
+    for (int m = 0; m <= g.mmax; ++m)
+        for (int l = m; l <= g.lmax; ++l, ++q) {
+            if (q >= g.npairs || g.pair_m[q] != m) return false;
+            for (int s = 0; s < (m ? 2 : 1); ++s) index[{l, m, s}] = k++;
+        }
+    if (q != g.npairs || k != g.ncoef) return false;
+    ob.L = std::max(3, g.lmax);
+    std::vector<int> sl, sm, ss;
+    switch (ob.L) {
+        case 3: orbit_stream<3>(sl, sm, ss); break;
+        case 4: orbit_stream<4>(sl, sm, ss); break;
+        case 5: orbit_stream<5>(sl, sm, ss); break;
+        default: orbit_stream<6>(sl, sm, ss); break;
+    }
+    const int nc = g.ncoef, N = int(sl.size()), st = psk::orb_stride(ob.L);
+    ob.n = g.nfac / 8;
+    ob.coef.assign(N, -1);
+    for (int j = 0; j < N; ++j) {
+        auto it = index.find({sl[j], sm[j], ss[j]});
+        if (it != index.end()) ob.coef[j] = it->second;
+    }
+    ob.pos.assign(g.nfac, -1);
+    ob.table.assign(size_t(ob.n + 1) * st, 0.0);
+    std::vector<double> scale(nc, 0.0);  // the size of each coefficient's cos/sin pair over the mesh
+    for (auto &kv : index) {
+        const auto [l, m, s] = kv.first;
+        for (int i = 0; i < g.nfac; ++i) {
+            const double v = std::fabs(g.dsph[size_t(i) * nc + kv.second]);
+            for (int s2 = 0; s2 < (m ? 2 : 1); ++s2) scale[index[{l, m, s2}]] = std::max(scale[index[{l, m, s2}]], v);
+        }
+    }
+    constexpr int kCos4[4] = {1, 0, -1, 0}, kSin4[4] = {0, 1, 0, -1};  // of multiples of 90 degrees
+    constexpr double kNorTol = 1e-14, kHarmTol = 1e-13;
+    int norb = 0;
+    for (int r = 0; r < g.nfac; ++r) {
+        const double *n = g.nor + 3 * r;
+        if (!(n[0] > 0 && n[1] > 0 && n[2] > 0)) continue;
+        if (norb == ob.n) return false;
+        double *row = &ob.table[size_t(norb) * st];
+        for (int c = 0; c < 3; ++c) row[c] = n[c];
+        const double *dr = g.dsph + size_t(r) * nc;
+        for (int j = 0; j < N; ++j) row[psk::kOrbHead + j] = ob.coef[j] >= 0 ? dr[ob.coef[j]] : 0.0;
+        double v[3] = {n[0], n[1], n[2]};
+        for (int t = 0; t < 4; ++t) {
+            for (int sg = 0; sg < 2; ++sg) {
+                int f = -1;
+                for (int i = 0; i < g.nfac && f < 0; ++i) {
+                    double d = 0;
+                    for (int c = 0; c < 3; ++c) d = std::max(d, std::fabs(g.nor[3 * i + c] - (sg ? -v[c] : v[c])));
+                    if (d <= kNorTol) f = i;
+                }
+                if (f < 0 || ob.pos[f] >= 0) return false;
+                ob.pos[f] = 8 * norb + 2 * t + sg;
+                for (auto &kv : index) {
+                    const auto [l, m, s] = kv.first;
+                    const double dc = dr[index[{l, m, 0}]], ds = m ? dr[index[{l, m, 1}]] : 0.0;
+                    const int c4 = kCos4[(m * t) & 3], s4 = kSin4[(m * t) & 3];
+                    double want = s ? ds * c4 + dc * s4 : dc * c4 - ds * s4;
+                    if (sg && (l & 1)) want = -want;
+                    if (!(std::fabs(g.dsph[size_t(f) * nc + kv.second] - want) <= kHarmTol * scale[kv.second])) return false;
+                }
+            }
+            const double x = v[0];
+            v[0] = -v[1];
+            v[1] = x;
+        }
+        ++norb;
+    }
+    if (norb != ob.n) return false;
+    // the correction rows: a member's harmonics minus the symmetric ones turned to it
+    std::vector<int> spos(nc, -1);
+    for (int j = 0; j < N; ++j)
+        if (ob.coef[j] >= 0) spos[ob.coef[j]] = j;
+    const int tiles = (N + 31) / 32;
+    ob.corr.assign(size_t(tiles) * (ob.n + 1) * 32 * 4, 0u);
+    for (int f = 0; f < g.nfac; ++f) {
+        const int o = ob.pos[f] / 8, mem = ob.pos[f] % 8, t = mem / 2, sg = mem % 2;
+        const double *row = &ob.table[size_t(o) * st + psk::kOrbHead];
+        for (auto &kv : index) {
+            const auto [l, m, s] = kv.first;
+            const double dc = row[spos[index[{l, m, 0}]]], ds = m ? row[spos[index[{l, m, 1}]]] : 0.0;
+            const int c4 = kCos4[(m * t) & 3], s4 = kSin4[(m * t) & 3];
+            double sym = s ? ds * c4 + dc * s4 : dc * c4 - ds * s4;
+            if (sg && (l & 1)) sym = -sym;
+            const int j = spos[kv.second];
+            unsigned &w = ob.corr[((size_t(j / 32) * (ob.n + 1) + o) * 32 + j % 32) * 4 + t];
+            w |= bf16_bits(g.dsph[size_t(f) * nc + kv.second] - sym) << (16 * sg);
+        }
+    }
+    // Dsph_0 = 1 is the brightness column
+    for (int i = 0; i < g.nfac; ++i)
+        if (g.dsph[size_t(i) * nc] != 1.0) return false;
+    return true;
+}
 }  // namespace
 
 // The per-workgroup buffers of ps_fit_batch_noalloc: a file-scope device array, one copy per GPU (held
@@ -180,6 +303,7 @@ struct ps_handle {
     // the J-free kernels (ps_fit2.h): FP64 fits and evaluations when every relative lightcurve fits
     // one pass; P2 holds the points in pass-schedule order
     bool v2 = false;
+    int orbit = 0;  // the OrbitModel of phase B (Lmax 3-6), 0: tiles
     DevProblem P2{};
     const DevProblem *dP2 = nullptr;
     Slots2 S2{};
@@ -258,6 +382,18 @@ int dispatch2(const Variant &v, F &&f) {
     return PS_ERR_UNSUPPORTED;
 }
 
+// Calls f.template operator()<Model>() for the handle's phase B of the J-free kernels.
+template <class F>
+int dispatch_model(const ps_handle *h, F &&f) {
+    switch (h->orbit) {
+        case 0: return dispatch2(h->var, [&]<int NT, int R>() { return f.template operator()<psk::TileModel<NT, R>>(); });
+        case 3: return f.template operator()<psk::OrbitModel<3>>();
+        case 4: return f.template operator()<psk::OrbitModel<4>>();
+        case 5: return f.template operator()<psk::OrbitModel<5>>();
+        default: return f.template operator()<psk::OrbitModel<6>>();
+    }
+}
+
 // The queue kernel's index of a coefficient layout (the order of its switch).
 int layout_id(const Variant &v) {
     if (v.nt == 1 && v.r == 0) return 0;
@@ -267,9 +403,9 @@ int layout_id(const Variant &v) {
     return 4;
 }
 
-template <int NT, int R, bool LS>
+template <class Model, bool LS>
 int launch_fit2(ps_handle *h, int grid, int nfits, double conw_r) {
-    hipLaunchKernelGGL((psk::fit_kernel2<NT, R, LS, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2, h->S2,
+    hipLaunchKernelGGL((psk::fit_kernel2<Model, LS, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2, h->S2,
                        h->d_freq, h->d_pole, nfits, conw_r, h->d_out);
     return hipGetLastError() == hipSuccess ? PS_OK : PS_ERR_DEVICE;
 }
@@ -582,6 +718,26 @@ extern "C" int ps_prepare(const ps_input *in, const ps_geometry *geo, int device
         Q.qperm = dev_upload(qperm.data(), nq, o);
         Q.fpos = dev_upload(fpos.data(), fpos.size(), o);
         Q.qsl = dev_upload(qsl.data(), nq, o);
+        Orbits ob;
+        if (build_orbits(*geo, ob)) {
+            h->orbit = ob.L;
+            const int ncol = psk::orb_ncoef(ob.L);
+            std::vector<int> scol(ncol), xcol;
+            int nsh = 0;  // fitted shape columns: 0 .. nsh - 1
+            for (int k = 0; k < ncoef; ++k) nsh += ia[k] != 0;
+            // a stream position without a fitted coefficient writes the last column of the row, which is
+            // past the residual then (c00, the only coefficient that can be fixed, is handled apart)
+            for (int j = 0; j < ncol; ++j) scol[j] = ob.coef[j] >= 0 && fpos[ob.coef[j]] >= 0 ? fpos[ob.coef[j]] : psk::kJP - 1;
+            for (int c = nsh; int(xcol.size()) < 7; ++c)
+                if (c != mfit) xcol.push_back(c);
+            Q.norb = ob.n;
+            Q.orb = dev_upload(ob.table.data(), ob.table.size(), o);
+            Q.ocorr = dev_upload(ob.corr.data(), ob.corr.size(), o);
+            Q.opos = dev_upload(ob.pos.data(), ob.pos.size(), o);
+            Q.scol = dev_upload(scol.data(), scol.size(), o);
+            Q.scoef = dev_upload(ob.coef.data(), ob.coef.size(), o);
+            Q.xcol = dev_upload(xcol.data(), xcol.size(), o);
+        }
         for (void *ptr : o)
             if (!ptr) return fail(ps_fail(PS_ERR_DEVICE, "device upload failed"));
         h->dP2 = dev_upload(&Q, 1, o);
@@ -602,8 +758,8 @@ extern "C" int ps_prepare(const ps_input *in, const ps_geometry *geo, int device
     h->nseg = nseg;
     if (h->v2) {
         int per_cu2 = 1;
-        dispatch2(h->var, [&]<int NT, int R>() {
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, psk::fit_kernel2<NT, R, false, kMaxFac>, psk::kWG2, 0);
+        dispatch_model(h, [&]<class Model>() {
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, psk::fit_kernel2<Model, false, kMaxFac>, psk::kWG2, 0);
             return 0;
         });
         h->slots2 = std::max(1, per_cu2) * prop.multiProcessorCount;
@@ -702,8 +858,8 @@ int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, d
     HIPCHECK(hipEventRecord(h->ev0, h->stream));
     if (use_v2(h)) {
         const int grid = std::min(nfits, h->slots2);
-        rc = dispatch2(h->var, [&]<int NT, int R>() {
-            return h->ls ? launch_fit2<NT, R, true>(h, grid, nfits, conw_r) : launch_fit2<NT, R, false>(h, grid, nfits, conw_r);
+        rc = dispatch_model(h, [&]<class Model>() {
+            return h->ls ? launch_fit2<Model, true>(h, grid, nfits, conw_r) : launch_fit2<Model, false>(h, grid, nfits, conw_r);
         });
     } else {
         const int grid = std::min(nfits, h->slots);
@@ -836,12 +992,12 @@ extern "C" int ps_fit_batch_noalloc(ps_handle *h, int nfits, const double *d_fre
         return ps_fail(PS_ERR_LIMIT, "ps_fit_batch_noalloc: %zu slots do not fit the scratch", slots);
     HIPCHECK(hipSetDevice(h->device));
     const int grid = int(std::min<size_t>(size_t(nfits), slots));
-    const int rc = dispatch2(h->var, [&]<int NT, int R>() {
+    const int rc = dispatch_model(h, [&]<class Model>() {
         if (h->ls)
-            hipLaunchKernelGGL((psk::fit_kernel2<NT, R, true, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream,
+            hipLaunchKernelGGL((psk::fit_kernel2<Model, true, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream,
                                h->dP2, T, d_freq, d_pole, nfits, conw_r, d_out);
         else
-            hipLaunchKernelGGL((psk::fit_kernel2<NT, R, false, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream,
+            hipLaunchKernelGGL((psk::fit_kernel2<Model, false, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream,
                                h->dP2, T, d_freq, d_pole, nfits, conw_r, d_out);
         return hipGetLastError() == hipSuccess ? PS_OK : PS_ERR_DEVICE;
     });
@@ -952,6 +1108,7 @@ struct ps_batch {
     int *d_counter = nullptr;
     Slots2 pool{};
     bool mixed = false;  // mixed precision: queue_kernel_mixed over the legacy problem descriptions
+    bool orbit = false;  // every problem has symmetry orbits: queue_kernel2<true, .>
     Slots lpool{};       // its per-slot buffers
     int slots = 0;
     psk::QueueJob *d_jobs = nullptr;
@@ -1010,17 +1167,19 @@ extern "C" int ps_batch_create(ps_handle *const *hs, int nh, ps_batch **out) {
     std::vector<int> layout(nh);
     size_t amax = 1, bmax = 1, fmax = 1, nptmax = 1, segmax = 1;
     b->cost.resize(nh);
+    b->orbit = !mixed;
+    for (int i = 0; i < nh; ++i) b->orbit = b->orbit && hs[i]->orbit != 0;
     for (int i = 0; i < nh; ++i) {
         const ps_handle *h = hs[i];
         probs[i] = mixed ? h->dP : h->dP2;
-        layout[i] = layout_id(h->var);
+        layout[i] = b->orbit ? h->orbit : layout_id(h->var);
         amax = std::max(amax, size_t(h->mfit) * h->mfit);
         bmax = std::max(bmax, size_t(h->mfit));
         fmax = std::max(fmax, size_t(h->nfac));
         nptmax = std::max(nptmax, size_t(h->npts));
         segmax = std::max(segmax, size_t(h->nseg));
         const double iters = h->P.n_iter_max > 0 ? h->P.n_iter_max : h->P.n_iter_min;
-        const double rows = mixed ? double(h->npts) : 16.0 * h->P2.pass_tile0[h->P2.npass];
+        const double rows = mixed ? double(h->npts) : double(h->P2.nsched);
         b->cost[i] = (iters + 1) * rows * (2.0 * h->nfac * h->ncoef + double(h->mfit) * (h->mfit + 1));
     }
     auto &o = b->owned;
@@ -1038,7 +1197,7 @@ extern "C" int ps_batch_create(ps_handle *const *hs, int nh, ps_batch **out) {
     if (mixed)
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, psk::queue_kernel_mixed<false>, kWG, 0);
     else
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, psk::queue_kernel2<false>, psk::kWG2, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, psk::queue_kernel2<true, false>, psk::kWG2, 0);
     b->slots = std::max(1, per_cu) * prop.multiProcessorCount;
     if (mixed) {
         Slots &L = b->lpool;
@@ -1152,13 +1311,14 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
                                    b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs + n0, n1, b->d_counter + 1,
                                    b->d_out);
         } else {
-            if (n0)
-                hipLaunchKernelGGL(psk::queue_kernel2<false>, dim3(std::min(n0, b->slots)), dim3(psk::kWG2), 0, b->stream,
-                                   b->d_probs, b->d_layout, b->d_conw, b->pool, b->d_jobs, n0, b->d_counter, b->d_out);
-            if (n1)
-                hipLaunchKernelGGL(psk::queue_kernel2<true>, dim3(std::min(n1, b->slots)), dim3(psk::kWG2), 0, b->stream,
-                                   b->d_probs, b->d_layout, b->d_conw, b->pool, b->d_jobs + n0, n1, b->d_counter + 1,
-                                   b->d_out);
+            auto launch = [&](auto *kern, int njob, const psk::QueueJob *job, int *counter) {
+                if (njob)
+                    hipLaunchKernelGGL(kern, dim3(std::min(njob, b->slots)), dim3(psk::kWG2), 0, b->stream, b->d_probs,
+                                       b->d_layout, b->d_conw, b->pool, job, njob, counter, b->d_out);
+            };
+            launch(b->orbit ? psk::queue_kernel2<true, false> : psk::queue_kernel2<false, false>, n0, b->d_jobs, b->d_counter);
+            launch(b->orbit ? psk::queue_kernel2<true, true> : psk::queue_kernel2<false, true>, n1, b->d_jobs + n0,
+                   b->d_counter + 1);
         }
         hipError_t e = hipStreamEndCapture(b->stream, &g);
         if (e == hipSuccess) e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
@@ -1234,8 +1394,8 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     HIPCHECK(hipEventRecord(h->ev0, h->stream));
     if (use_v2(h)) {
         const int grid = std::min(nvec, h->slots2);
-        rc = dispatch2(h->var, [&]<int NT, int R>() {
-            hipLaunchKernelGGL((psk::eval_kernel2<NT, R, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2,
+        rc = dispatch_model(h, [&]<class Model>() {
+            hipLaunchKernelGGL((psk::eval_kernel2<Model, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2,
                                h->S2, E.a, nvec, conw_r, d_al, d_be, d_ch, d_y, d_dy);
             return hipGetLastError() == hipSuccess ? PS_OK : PS_ERR_DEVICE;
         });

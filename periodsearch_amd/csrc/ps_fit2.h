@@ -9,9 +9,10 @@
 // walks the points in passes of at most 8 tiles of 16 points, built on the host so that every
 // relative lightcurve lies inside one pass (the reference, too, holds one lightcurve's rows at a
 // time: dytemp, mrqcof.c:23, 51-104).  Per pass:
-//  B  model rows (bright.c:14-126, conv.c:12-29): each wave runs the MFMA facet loop of ps_kernels.h
-//     over its two tiles and writes the fitted columns of the raw rows into LDS, plus the model value
-//     of a relative point, or the residual y - ymod of a calibrated one;
+//  B  model rows (bright.c:14-126, conv.c:12-29): the fitted columns of the raw rows into LDS, plus the
+//     model value of a relative point, or the residual y - ymod of a calibrated one; by symmetry orbits
+//     of the facets (ps_orbit.h), or, on a mesh without them, by the MFMA facet loop of ps_kernels.h
+//     over two tiles a wave;
 //  C  for every relative lightcurve of the pass (one wave each): the column sums dave and ave, then
 //     the normalisation of its rows in place (mrqcof.c:89-101) and the residual y - coef*ymod;
 //  D  the weighted Gram matrix of the pass's normalised rows plus the residual column on
@@ -22,6 +23,7 @@
 #pragma once
 
 #include "ps_kernels.h"
+#include "ps_orbit.h"
 
 namespace psk {
 
@@ -38,13 +40,20 @@ struct Shared2 {
     double a[64];     // parameters under evaluation
     double cg[64];    // accepted parameters
     double atry[64];
-    double nx[NFM], ny[NFM], nz[NFM], acl[NFM], acls[NFM];  // normals, Area*cl, Area*cls
+    double nx[NFM], ny[NFM], nz[NFM];  // normals
+    union {
+        struct {
+            double acl[NFM], acls[NFM];  // tile form: Area*cl, Area*cls
+        };
+        orb_d2 tab[NFM + 8];             // orbit form: (Area*cl, Area*cls) by orbit, then eight zeros
+    };
     union {
         double da[64];       // the LM step: the Gauss-Jordan right-hand side, then its solution
         double csum[2][64];  // phase C: the column sums of two consecutive lightcurves
     };
-    double bl[9], dbl[18], hbl[18];  // pole rotation, its derivatives, the pole-frame generators
+    double bl[9], hbl[18];  // pole rotation, the pole-frame generators of its derivatives
     double scal[4];
+    double ascale, amax[kWaves2];  // orbit form: the power of two the table is scaled by, each wave's largest entry
     int job;  // the queue kernel: the job claimed by the workgroup
     union {
         double rows[kPassRows * kJP];  // the pass's Jacobian rows (fitted columns + residual)
@@ -76,6 +85,50 @@ __device__ inline void curv2(const DevProblem &P, const double *a, Shared2<NFM> 
         sh.acl[i] = ar * cl;
         sh.acls[i] = ar * cls;
     }
+}
+
+// The same into the orbit form's table: facet i's entry, negated for the member -n_k of its pair.  With
+// LS the second number is Area (the loop multiplies it by cls and sums the Lambert columns from it).  The
+// table is scaled by a power of two so that its largest number is about 1 (a runaway Lambert weight or
+// shape would leave the range of the correction's FP32); the row sums are scaled back by sh.ascale.
+template <bool LS, int NFM>
+__device__ inline void curv_orbit(const DevProblem &P, const double *a, Shared2<NFM> &sh, double *area) {
+    constexpr int kPer = (NFM + kWG2 - 1) / kWG2;  // facets per lane
+    const double cl = exp(a[P.nc + 6]), cls = a[P.nc + 7];
+    double t0[kPer], t1[kPer], big = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = threadIdx.x + k * kWG2;
+        t0[k] = t1[k] = 0;
+        if (i < P.nf) {
+            const double ar = gload(P.darea, i) * exp(facet_shape_sum(P, a, i));
+            area[i] = ar;
+            t0[k] = ar * cl;
+            t1[k] = LS ? ar : ar * cls;
+        }
+        big = fmax(big, fmax(fabs(t0[k]), fabs(t1[k])));
+    }
+    big = fmax(big, dpp<0xB1>(big));
+    big = fmax(big, dpp<0x4E>(big));
+    big = fmax(big, dpp<0x141>(big));
+    big = fmax(big, dpp<0x140>(big));
+    big = pair_max(pair_max(big, false), true);
+    if ((threadIdx.x & 63) == 0) sh.amax[threadIdx.x >> 6] = big;
+    __syncthreads();
+    big = fmax(fmax(sh.amax[0], sh.amax[1]), fmax(sh.amax[2], sh.amax[3]));
+    const int ex = (big > 0 && big < __builtin_inf()) ? max(-1000, min(1000, ilogb(big))) : 0;
+    const double inv = ldexp(1.0, -ex);
+    if (threadIdx.x == 0) sh.ascale = ldexp(1.0, ex);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = threadIdx.x + k * kWG2;
+        if (i < P.nf) {
+            const int pos = gload(P.opos, i);
+            const double f = (pos & 1) ? -inv : inv;
+            sh.tab[pos] = orb_d2{t0[k] * f, t1[k] * f};
+        }
+    }
+    if (threadIdx.x < 8) sh.tab[8 * P.norb + threadIdx.x] = orb_d2{0, 0};
 }
 
 __device__ inline double wave_sum(double x) {  // sum over the 64 lanes, the same bits in every lane
@@ -115,6 +168,57 @@ __device__ inline void facet_sums_n(const double *area, const double *nx, const 
     s[0] = wave_sum(s0);
     s[1] = wave_sum(s1);
     s[2] = wave_sum(s2);
+}
+
+// The three convexity rows (conv.c:12-29) of the last pass: res_c = sum Area*n_c, dres_k = sum
+// Area*Dsph_k*n_c; lane (k, q) sums coefficient k (k == nc: the plain sums) over facets q, q+4, ..., the
+// quarters are added across the lane quad.  Their residual is 0 - res_c (y = 0).  The rows' places have
+// been written as model rows before: every column is rewritten here, after all waves are done.
+template <int NFM>
+__device__ __forceinline__ void conv_rows2(const DevProblem &P, Shared2<NFM> &sh, int tile0, const double *area,
+                                           double *raw_y, double *raw_dyda) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nc = P.nc, pitch = P.dpitch, mfit = P.mfit, ma = P.ma;
+    const int q4 = lane & 3, k = wave * 16 + (lane >> 2);
+    double s0 = 0, s1 = 0, s2 = 0;
+    if (k <= nc) {
+#pragma unroll 4
+        for (int i = q4; i < P.nf; i += 4) {
+            const double t = gload(area, i) * (k < nc ? gload(P.dsph, i * pitch + k) : 1.0);
+            s0 += t * sh.nx[i];
+            s1 += t * sh.ny[i];
+            s2 += t * sh.nz[i];
+        }
+    }
+    s0 += dpp<0xB1>(s0);
+    s1 += dpp<0xB1>(s1);
+    s2 += dpp<0xB1>(s2);
+    s0 += dpp<0x4E>(s0);
+    s1 += dpp<0x4E>(s1);
+    s2 += dpp<0x4E>(s2);
+    const int r0 = P.conv_q - tile0 * 16;
+    const double sv[3] = {s0, s1, s2};
+    if (q4 == 0 && k <= nc) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            double *row = sh.u.rows + (r0 + c) * kJP;
+            if (k < nc) {
+                const int col = P.fpos[k];
+                if (col >= 0) row[col] = sv[c];
+                if (raw_dyda) raw_dyda[size_t(P.npts - 3 + c) * ma + k] = sv[c];
+            } else {
+                row[mfit] = 0.0 - sv[c];
+                if (raw_dyda) raw_y[P.npts - 3 + c] = sv[c];
+            }
+        }
+    }
+    // the other parameters' columns of the convexity rows are zero
+    for (int it = threadIdx.x; it < 3 * (ma - nc); it += kWG2) {
+        const int c = it / (ma - nc), kk = nc + it - c * (ma - nc);
+        const int col = P.fpos[kk];
+        if (col >= 0) sh.u.rows[(r0 + c) * kJP + col] = 0.0;
+        if (raw_dyda) raw_dyda[size_t(P.npts - 3 + c) * ma + kk] = 0.0;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -348,53 +452,164 @@ __device__ __forceinline__ void model_rows2(const DevProblem &P, Shared2<NFM> &s
     else if (tl < ntl)
         tiles.template operator()<1>();
     if (last) {
-        // convexity rows (conv.c:12-29): res_c = sum Area*n_c, dres_k = sum Area*Dsph_k*n_c; lane (k, q)
-        // sums coefficient k (k == nc: the plain sums) over facets q, q+4, ..., the quarters are added
-        // across the lane quad.  Their residual is 0 - res_c (y = 0).  The tile that holds them has
-        // written model rows there too: every column is rewritten here, after all waves are done.
         __syncthreads();
-        const int q4 = lane & 3, k = wave * 16 + (lane >> 2);
-        double s0 = 0, s1 = 0, s2 = 0;
-        if (k <= nc) {
-#pragma unroll 4
-            for (int i = q4; i < P.nf; i += 4) {
-                const double t = gload(area, i) * (k < nc ? gload(P.dsph, i * pitch + k) : 1.0);
-                s0 += t * sh.nx[i];
-                s1 += t * sh.ny[i];
-                s2 += t * sh.nz[i];
-            }
-        }
-        s0 += dpp<0xB1>(s0);
-        s1 += dpp<0xB1>(s1);
-        s2 += dpp<0xB1>(s2);
-        s0 += dpp<0x4E>(s0);
-        s1 += dpp<0x4E>(s1);
-        s2 += dpp<0x4E>(s2);
-        const int r0 = P.conv_q - tile0 * 16;
-        const double sv[3] = {s0, s1, s2};
-        if (q4 == 0 && k <= nc) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                double *row = sh.u.rows + (r0 + c) * kJP;
-                if (k < nc) {
-                    const int col = P.fpos[k];
-                    if (col >= 0) row[col] = sv[c];
-                    if (raw_dyda) raw_dyda[size_t(P.npts - 3 + c) * ma + k] = sv[c];
-                } else {
-                    row[mfit] = 0.0 - sv[c];
-                    if (raw_dyda) raw_y[P.npts - 3 + c] = sv[c];
-                }
-            }
-        }
-        // the other parameters' columns of the convexity rows are zero
-        for (int it = threadIdx.x; it < 3 * (ma - nc); it += kWG2) {
-            const int c = it / (ma - nc), kk = nc + it - c * (ma - nc);
-            const int col = P.fpos[kk];
-            if (col >= 0) sh.u.rows[(r0 + c) * kJP + col] = 0.0;
-            if (raw_dyda) raw_dyda[size_t(P.npts - 3 + c) * ma + kk] = 0.0;
-        }
+        conv_rows2(P, sh, tile0, area, raw_y, raw_dyda);
     }
 }
+
+// ---------------------------------------------------------------------------------------------
+// Phase B of one pass by symmetry orbits (ps_orbit.h): lane l of the two waves of group g owns pass row
+// 64g + l.  Each of the two sums its half of the orbits; they exchange through the row's own LDS
+// columns (once neither needs its buffer of X there any more): the first hands over its odd-l sums, the second its even-l sums and the six rotation sums,
+// and after a barrier the first completes the even-l columns and everything else of the row, the
+// second the odd-l columns.  The roles alternate with the pass, so that the longer epilogue falls on
+// every SIMD in turn.  A group with no row in the pass only joins the barrier.
+// ---------------------------------------------------------------------------------------------
+template <int L, bool LS, int NFM>
+__device__ __forceinline__ void model_rows_orbit(const DevProblem &P, Shared2<NFM> &sh, int tile0, int ntl, int turn,
+                                                 bool last, const double *area, double *raw_y, double *raw_dyda) {
+    constexpr OrbLayout<L> lay{};
+    constexpr int N = orb_ncoef(L);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = wave >> 1, half = (wave ^ turn) & 1;
+    const int nc = P.nc, mfit = P.mfit, ma = P.ma, norb = P.norb;
+    const double *a = sh.a;
+    const bool on = 4 * g < ntl;
+    const int q = tile0 * 16 + 64 * g + lane;  // the point arrays run a whole pass past the schedule
+    double *row = sh.u.rows + (64 * g + lane) * kJP;
+    double e[3], e0[3], sf = 0, cf = 0, eph = 0;
+    OrbAcc<L, LS> A;
+    // the brightness sum's hand-over column: the c00 column, or the residual's where c00 is fixed
+    const int c0 = P.c00col >= 0 ? P.c00col : mfit;
+    if (on) {
+        {
+            double rot[3];
+            point_dirs(P, a, q, sh, e, e0, rot);
+            sf = rot[0];
+            cf = rot[1];
+            eph = exp(-gload(P.alpha, q) / a[nc + 4]);
+        }
+        const int mid = (norb + 1) >> 1, end = half ? norb : mid;
+        char *xw = reinterpret_cast<char *>(sh.u.rows + 64 * g * kJP) + half * kXBytes;
+        A.clear();
+        for (int o = half ? mid : 0; o < end; o += kSegOrbits) {
+            const int cnt = min(kSegOrbits, end - o);
+            orbit_loop<L, LS>(P.orb, o, o + cnt, sh.tab, 128 * norb, LS ? a[nc + 7] : 0.0, e, e0, xw + lane * 16, A);
+            orbit_correct<L, LS>(reinterpret_cast<const orb_u4 *>(P.ocorr), norb, o, cnt, xw, A);
+        }
+    }
+    __syncthreads();  // the buffers of X lie in the rows
+    if (on) {
+        if (half == 0) {
+#pragma unroll
+            for (int j = lay.neven; j < N; ++j) row[uload(P.scol, j)] = A.c[j];
+        } else {
+            row[c0] = A.c[0];
+#pragma unroll
+            for (int j = 1; j < lay.neven; ++j) row[uload(P.scol, j)] = A.c[j];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                row[uload(P.xcol, k)] = A.S[k];
+                row[uload(P.xcol, 3 + k)] = A.U[k];
+            }
+            if constexpr (LS) {
+                row[uload(P.xcol, 6)] = A.d1;
+                sh.csum[g][lane] = A.d2;
+            }
+        }
+    }
+    __syncthreads();
+    if (on) {
+        const double p1 = a[nc + 3], p2 = a[nc + 4], al = gload(P.alpha, q);
+        double dphp[3];
+        const double asc = sh.ascale, phs = phase_scale(a, nc, al, eph, p1 * eph * al / (p2 * p2), dphp);
+        const double scale = phs * asc;
+        const int orig = raw_dyda ? gload(P.qperm, q) : -1;
+        double *rraw = raw_dyda + size_t(orig >= 0 ? orig : 0) * ma;
+        auto shape = [&](int j) {  // a coefficient's column, complete
+            const int col = uload(P.scol, j);
+            const double v = scale * (half == 0 ? A.c[j] + row[col] : row[col] + A.c[j]);
+            row[col] = v;
+            if (orig >= 0) {
+                const int k = uload(P.scoef, j);
+                if (k >= 0) rraw[k] = v;
+            }
+        };
+        if (half) {
+#pragma unroll
+            for (int j = lay.neven; j < N; ++j) shape(j);
+        } else {
+            const double br = (A.c[0] + row[c0]) * asc;
+#pragma unroll
+            for (int j = 1; j < lay.neven; ++j) shape(j);
+            double S[3], U[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                S[k] = A.S[k] + row[uload(P.xcol, k)];
+                U[k] = A.U[k] + row[uload(P.xcol, 3 + k)];
+            }
+            constexpr int kOther = 8;  // beta/lambda/omega, 3 phase, cl, cls
+            double ov[kOther];
+            {
+                double js[3];
+                const double rot[3] = {sf, cf, gload(P.t, q)};
+                spin_columns(sh, e, e0, rot, S, U, js);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) ov[k] = scale * js[k];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) ov[3 + i] = br * dphp[i];
+                ov[6] = LS ? scale * (A.d1 + row[uload(P.xcol, 6)]) * exp(a[nc + 6]) : 0.0;
+                ov[7] = LS ? scale * (A.d2 + sh.csum[g][lane]) : 0.0;
+            }
+            const double ymod = br * phs;
+            if (P.c00col >= 0) row[P.c00col] = ymod;  // Dsph_0 = 1 on every facet
+#pragma unroll
+            for (int k = 0; k < kOther; ++k) {
+                const int c = uload(P.fpos, nc + k);
+                if (c >= 0) row[c] = ov[k];
+            }
+            // relative point: the model value (phase C normalises it); calibrated: the residual
+            row[mfit] = gload(P.qrel, q) ? ymod : gload(P.y, q) - ymod;
+            if (orig >= 0) {
+                raw_y[orig] = ymod;
+                rraw[0] = ymod;
+#pragma unroll
+                for (int k = 0; k < kOther; ++k) rraw[nc + k] = ov[k];
+            }
+        }
+    }
+    if (last) {
+        __syncthreads();
+        conv_rows2(P, sh, tile0, area, raw_y, raw_dyda);
+    }
+}
+
+// The two forms of phase B: tiles on MFMA for any mesh and coefficient set, orbits for the symmetric
+// meshes of trifac.c with degree and order up to 6.
+template <int NT_, int R_>
+struct TileModel {
+    template <bool LS, int NFM>
+    __device__ static __forceinline__ void curv(const DevProblem &P, const double *a, Shared2<NFM> &sh, double *area) {
+        curv2(P, a, sh, area);
+    }
+    template <bool LS, int NFM>
+    __device__ static __forceinline__ void rows(const DevProblem &P, Shared2<NFM> &sh, int tile0, int ntl, int k, bool last,
+                                                const double *area, double *raw_y, double *raw_dyda) {
+        model_rows2<NT_, R_, LS>(P, sh, tile0, ntl, k & 3, last, area, raw_y, raw_dyda);
+    }
+};
+template <int L_>
+struct OrbitModel {
+    template <bool LS, int NFM>
+    __device__ static __forceinline__ void curv(const DevProblem &P, const double *a, Shared2<NFM> &sh, double *area) {
+        curv_orbit<LS>(P, a, sh, area);
+    }
+    template <bool LS, int NFM>
+    __device__ static __forceinline__ void rows(const DevProblem &P, Shared2<NFM> &sh, int tile0, int ntl, int k, bool last,
+                                                const double *area, double *raw_y, double *raw_dyda) {
+        model_rows_orbit<L_, LS>(P, sh, tile0, ntl, k & 1, last, area, raw_y, raw_dyda);
+    }
+};
 
 // Per-row data of a pass for phases C and D, loaded once after phase B (the loads overlap the barrier):
 // lane i holds pass rows i and 64 + i.  y: the observation, sl: sig*Lpoints of a relative point
@@ -646,12 +861,12 @@ __device__ __forceinline__ void stash_io(int nb, int ow, Prec<false>::V4 acc[kOw
 // mrqcof for the parameters in sh.a: alpha[mfit][mfit], beta[mfit] to the given buffers, chi2
 // returned.  raw_y / raw_dyda: the raw rows (ps_eval).
 // ---------------------------------------------------------------------------------------------
-template <int NT, int R, bool LS, int NFM>
+template <class Model, bool LS, int NFM>
 __device__ __forceinline__ double mrqcof2(const DevProblem &P, Shared2<NFM> &sh, double wqc, double *area,
                                           double *stash, double *alpha, double *beta, double *raw_y,
                                           double *raw_dyda) {
     using Pd = Prec<false>;
-    curv2(P, sh.a, sh, area);
+    Model::template curv<LS>(P, sh.a, sh, area);
     blmatrix_lds(sh.a[P.nc], sh.a[P.nc + 1], sh);
     __syncthreads();
     const int npass = P.npass;
@@ -665,7 +880,7 @@ __device__ __forceinline__ double mrqcof2(const DevProblem &P, Shared2<NFM> &sh,
         // latency-bound phase (lightcurve sums, Gram, Gauss-Jordan), its instructions go first and the
         // facet loop fills the gaps
         __builtin_amdgcn_s_setprio(0);
-        model_rows2<NT, R, LS>(P, sh, tile0, ntl, k & 3, last, area, raw_y, raw_dyda);
+        Model::template rows<LS>(P, sh, tile0, ntl, k, last, area, raw_y, raw_dyda);
         __builtin_amdgcn_s_setprio(2);
         const PassRowData rd = load_pass_rows(P, tile0, wqc);
         __syncthreads();
@@ -813,7 +1028,7 @@ __device__ inline SlotPtrs slot_ptrs(const Slots2 &S, int slot) {
     return p;
 }
 
-template <int NT, int R, bool LS, int NFM>
+template <class Model, bool LS, int NFM>
 __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, const SlotPtrs &sp, double freq,
                                         int pole, double conw_r, ps_fit_result *out) {
     const int tid = threadIdx.x;
@@ -919,7 +1134,7 @@ __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, c
             __syncthreads();
             // the starting point fills the current buffers, a trial point the other ones
             const bool other = !init;
-            const double chi = uniform_double(mrqcof2<NT, R, LS>(P, sh, wqc, area, sp.stash,
+            const double chi = uniform_double(mrqcof2<Model, LS>(P, sh, wqc, area, sp.stash,
                                                                  (cur ^ other) ? sp.alpha1 : sp.alpha0,
                                                                  (cur ^ other) ? sp.beta1 : sp.beta0, nullptr, nullptr));
             if (init) {
@@ -951,7 +1166,7 @@ __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, c
             __syncthreads();
             // curv(cg) (period_search_BOINC.cpp:874); after an accepted step cg is the trial point, whose
             // areas the evaluation has just computed from the same bits
-            if (!__builtin_amdgcn_readfirstlane(fresh)) curv2(P, sh.a, sh, area);
+            if (!__builtin_amdgcn_readfirstlane(fresh)) Model::template curv<LS>(P, sh.a, sh, area);
             __syncthreads();
             if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
                 double sn[3];
@@ -996,14 +1211,14 @@ __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, c
 }
 
 // The fits of one problem, a grid-stride loop over them.
-template <int NT, int R, bool LS, int NFM>
+template <class Model, bool LS, int NFM>
 __global__ __launch_bounds__(kWG2, 2) void fit_kernel2(const DevProblem *__restrict__ Pp, Slots2 S, const double *freq,
                                                        const int *pole, int nfits, double conw_r, ps_fit_result *out) {
     const DevProblem &P = *Pp;
     __shared__ Shared2<NFM> sh;
     const SlotPtrs sp = slot_ptrs(S, blockIdx.x);
     load_facets2(P, sh);
-    for (int fi = blockIdx.x; fi < nfits; fi += gridDim.x) fit_one<NT, R, LS>(P, sh, sp, freq[fi], pole[fi], conw_r, out + fi);
+    for (int fi = blockIdx.x; fi < nfits; fi += gridDim.x) fit_one<Model, LS>(P, sh, sp, freq[fi], pole[fi], conw_r, out + fi);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1035,7 +1250,8 @@ struct QueueJob {
     int pad;
 };
 
-template <bool LS>
+// ORBIT: every problem of the batch has symmetry orbits (the layout is then its OrbitModel's, Lmax 3-6).
+template <bool ORBIT, bool LS>
 __global__ __launch_bounds__(kWG2, 2) void queue_kernel2(const DevProblem *const *probs, const int *layout,
                                                          const double *conw, Slots2 S, const QueueJob *jobs, int njobs,
                                                          int *counter, ps_fit_result *out) {
@@ -1058,12 +1274,22 @@ __global__ __launch_bounds__(kWG2, 2) void queue_kernel2(const DevProblem *const
             prev = prob;
         }
         const double cw = conw[prob];
-        switch (__builtin_amdgcn_readfirstlane(layout[prob])) {
-            case 0: fit_one<1, 0, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
-            case 1: fit_one<1, 9, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
-            case 2: fit_one<2, 4, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
-            case 3: fit_one<3, 1, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
-            default: fit_one<4, 0, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+        const int lay = __builtin_amdgcn_readfirstlane(layout[prob]);
+        if constexpr (ORBIT) {
+            switch (lay) {
+                case 3: fit_one<OrbitModel<3>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                case 4: fit_one<OrbitModel<4>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                case 5: fit_one<OrbitModel<5>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                default: fit_one<OrbitModel<6>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+            }
+        } else {
+            switch (lay) {
+                case 0: fit_one<TileModel<1, 0>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                case 1: fit_one<TileModel<1, 9>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                case 2: fit_one<TileModel<2, 4>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                case 3: fit_one<TileModel<3, 1>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+                default: fit_one<TileModel<4, 0>, LS>(P, sh, sp, freq, pole, cw, out + oi); break;
+            }
         }
     }
 }
@@ -1111,7 +1337,7 @@ __global__ void queue_reset(int *counter, int n) {
 }
 
 // mrqcof for externally supplied parameter vectors (ps_eval), J-free.
-template <int NT, int R, int NFM>
+template <class Model, int NFM>
 __global__ __launch_bounds__(kWG2, 2) void eval_kernel2(const DevProblem *__restrict__ Pp, Slots2 S, const double *avec,
                                                      int nvec, double conw_r, double *alpha, double *beta,
                                                      double *chisq, double *raw_y, double *raw_dyda) {
@@ -1125,7 +1351,7 @@ __global__ __launch_bounds__(kWG2, 2) void eval_kernel2(const DevProblem *__rest
     for (int v = blockIdx.x; v < nvec; v += gridDim.x) {
         if (tid < P.ma) sh.a[tid] = avec[size_t(v) * P.ma + tid];
         __syncthreads();
-        const double c = mrqcof2<NT, R, true>(P, sh, conv_weight(conw_r), area, stash, al, be,
+        const double c = mrqcof2<Model, true>(P, sh, conv_weight(conw_r), area, stash, al, be,
                                                   raw_y ? raw_y + size_t(v) * P.npts : nullptr,
                                                   raw_dyda ? raw_dyda + size_t(v) * P.npts * P.ma : nullptr);
         for (int it = tid; it < mfit * mfit; it += kWG2)

@@ -81,6 +81,14 @@ struct DevProblem {
     const int *qperm;  // [nsched] the point's index in input order (-1: padding)
     const int *fpos;   // [ma] the row column of a parameter (-1: fixed); column mfit = the residual
     const double *qsl; // [nsched] sig*Lpoints of a relative lightcurve's point (mrqcof.c:94), else 0
+    // Symmetry orbits of the facets (ps_orbit.h; norb = 0: the mesh has none).  orb: a row per orbit and
+    // one more; opos[f]: facet f's entry in the kernels' area table, 8 * orbit + 2k + (1: -n_k);
+    // scol / scoef: the row column / coefficient of each stream position; xcol: eight row columns
+    // that hold no shape coefficient and not the residual.
+    int norb;
+    const double *orb;
+    const unsigned *ocorr;  // the correction rows, bfloat16 pairs
+    const int *opos, *scol, *scoef, *xcol;
 };
 
 struct Slots {
@@ -237,7 +245,8 @@ __device__ inline void blmatrix_lds(double bet, double lam, SH &sh) {
         double bl[3][3], dbl[2][3][3];
         blmatrix(bet, lam, bl, dbl);
         for (int i = 0; i < 9; ++i) sh.bl[i] = bl[i / 3][i % 3];
-        for (int i = 0; i < 18; ++i) sh.dbl[i] = dbl[i / 9][(i / 3) % 3][i % 3];
+        if constexpr (requires { sh.dbl; })
+            for (int i = 0; i < 18; ++i) sh.dbl[i] = dbl[i / 9][(i / 3) % 3][i % 3];
         for (int j = 0; j < 2; ++j)
             for (int i = 0; i < 3; ++i)
                 for (int k = 0; k < 3; ++k)
