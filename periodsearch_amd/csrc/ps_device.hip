@@ -23,6 +23,7 @@
 #include "ps_internal.h"
 #include "ps_kernels.h"
 #include "ps_fit2.h"
+#include "ps_spread.h"
 
 using psk::DevProblem;
 using psk::Slots;
@@ -140,8 +141,8 @@ bool build_schedule(const std::vector<int> &lc_start, const std::vector<int> &lc
     return true;
 }
 
-// The symmetry orbits of a geometry (ps_orbit.h): for every orbit the representative's normal and
-// harmonics, for every facet its entry (8 * orbit + 2k + (1: -n_k)).  Returns false where the mesh or the
+// The symmetry orbits of a geometry (ps_orbit.h): for every orbit the members' mean normal (they differ by
+// a few 1e-16, their own rounding) and the representative's harmonics, for every facet its entry (8 * orbit + 2k + (1: -n_k)).  Returns false where the mesh or the
 // coefficient set is not of that kind (a caller may fill ps_geometry itself); every member's normal and
 // harmonics are compared with what the symmetry gives, to a few units of rounding.
 struct Orbits {
@@ -207,10 +208,10 @@ bool build_orbits(const ps_geometry &g, Orbits &ob) {
         if (!(n[0] > 0 && n[1] > 0 && n[2] > 0)) continue;
         if (norb == ob.n) return false;
         double *row = &ob.table[size_t(norb) * st];
-        for (int c = 0; c < 3; ++c) row[c] = n[c];
         const double *dr = g.dsph + size_t(r) * nc;
         for (int j = 0; j < N; ++j) row[psk::kOrbHead + j] = ob.coef[j] >= 0 ? dr[ob.coef[j]] : 0.0;
         double v[3] = {n[0], n[1], n[2]};
+        long double mean[3] = {0, 0, 0};  // of the members' normals, turned back to the representative
         for (int t = 0; t < 4; ++t) {
             for (int sg = 0; sg < 2; ++sg) {
                 int f = -1;
@@ -221,6 +222,10 @@ bool build_orbits(const ps_geometry &g, Orbits &ob) {
                 }
                 if (f < 0 || ob.pos[f] >= 0) return false;
                 ob.pos[f] = 8 * norb + 2 * t + sg;
+                const long double x = sg ? -g.nor[3 * f] : g.nor[3 * f], y = sg ? -g.nor[3 * f + 1] : g.nor[3 * f + 1];
+                mean[0] += x * kCos4[t] + y * kSin4[t];
+                mean[1] += y * kCos4[t] - x * kSin4[t];
+                mean[2] += sg ? -g.nor[3 * f + 2] : g.nor[3 * f + 2];
                 for (auto &kv : index) {
                     const auto [l, m, s] = kv.first;
                     const double dc = dr[index[{l, m, 0}]], ds = m ? dr[index[{l, m, 1}]] : 0.0;
@@ -234,6 +239,7 @@ bool build_orbits(const ps_geometry &g, Orbits &ob) {
             v[0] = -v[1];
             v[1] = x;
         }
+        for (int c = 0; c < 3; ++c) row[c] = double(mean[c] / 8);
         ++norb;
     }
     if (norb != ob.n) return false;
@@ -287,6 +293,21 @@ int noalloc_setup(int device) {
 }
 }  // namespace
 
+namespace {
+// Device buffers of the spread form (ps_spread.h), one allocation kept by a handle or batch and grown on
+// demand.  The passes in flight are bounded: longer job lists run in pieces.
+constexpr int kSpreadPasses = 8192;  // 192 MiB of Gram blocks
+struct Spread {
+    psk::SpreadBuf B{};
+    psk::SpreadJob *jobs = nullptr;
+    psk::SpreadTask *tasks = nullptr;
+    std::vector<psk::SpreadJob> hjobs;  // host copies, alive until their uploads have run
+    std::vector<psk::SpreadTask> htasks;
+    char *arena = nullptr;
+    size_t cap = 0;
+};
+}  // namespace
+
 struct ps_handle {
     int device = 0;
     int precision = PS_FP64;
@@ -314,6 +335,7 @@ struct ps_handle {
         double *a = nullptr, *al = nullptr, *be = nullptr, *ch = nullptr, *y = nullptr, *dy = nullptr;
         size_t ca = 0, cal = 0, cbe = 0, cch = 0, cy = 0, cdy = 0;
     } ev;
+    Spread spread;
     std::vector<double> wq2_host;
     double *d_wq2 = nullptr;
     std::vector<void *> owned;
@@ -805,6 +827,137 @@ int ensure_scratch(ps_handle *h, bool v2) {
 }
 }  // namespace
 
+// ---------------------------------------------------------------------------------------------
+// The spread form (ps_spread.h): host side.
+// ---------------------------------------------------------------------------------------------
+namespace {
+// Time of one evaluation of the jobs with q passes to a task, in units of a pass on a CU of its own: a task
+// also forms its own areas (kSpreadSetup), and two workgroups on a CU take 1.5 times as long as one.
+constexpr double kSpreadSetup = 0.4, kSpreadPaired = 1.5;
+double spread_time(const std::vector<psk::SpreadJob> &jobs, int q, int slots) {
+    long tasks = 0;
+    int longest = 0;
+    for (const auto &j : jobs) {
+        tasks += (j.npass + q - 1) / q;
+        longest = std::max(longest, std::min(q, j.npass));
+    }
+    const double per = longest + kSpreadSetup;
+    return tasks <= slots / 2 ? per : kSpreadPaired * double((tasks + slots - 1) / slots) * per;
+}
+
+std::vector<psk::SpreadTask> spread_tasks(const std::vector<psk::SpreadJob> &jobs, int slots) {
+    int longest = 1, best = 1;
+    for (const auto &j : jobs) longest = std::max(longest, j.npass);
+    for (int q = 2; q <= longest; ++q)
+        if (spread_time(jobs, q, slots) < spread_time(jobs, best, slots)) best = q;
+    std::vector<psk::SpreadTask> tasks;
+    for (int j = 0; j < int(jobs.size()); ++j) {
+        const int np = jobs[j].npass, n = (np + best - 1) / best;  // tasks of equal length, give or take a pass
+        for (int i = 0; i < n; ++i) tasks.push_back({j, int(long(np) * i / n), int(long(np) * (i + 1) / n)});
+    }
+    std::stable_sort(tasks.begin(), tasks.end(), [](const psk::SpreadTask &x, const psk::SpreadTask &y) {
+        return x.k1 - x.k0 > y.k1 - y.k0;
+    });
+    return tasks;
+}
+
+// Buffers for a piece of jobs; false when memory runs out.
+bool spread_buffers(Spread &S, size_t njobs, size_t ntasks, size_t passes, size_t mfit, size_t nfac) {
+    size_t need = 0;
+    auto place = [&](size_t bytes) {
+        const size_t at = need;
+        need += (bytes + 255) & ~size_t(255);
+        return at;
+    };
+    S.B.a_stride = mfit * mfit;
+    S.B.b_stride = mfit;
+    S.B.f_stride = nfac;
+    const size_t state = place(njobs * sizeof(psk::SpreadState)), part = place(passes * psk::kStashPerSlot * sizeof(double)),
+                 alpha = place(2 * njobs * S.B.a_stride * sizeof(double)), beta = place(2 * njobs * S.B.b_stride * sizeof(double)),
+                 area = place(2 * njobs * S.B.f_stride * sizeof(double)), done = place(sizeof(int)),
+                 jobs = place(njobs * sizeof(psk::SpreadJob)), tasks = place(ntasks * sizeof(psk::SpreadTask));
+    if (need > S.cap) {
+        (void)hipFree(S.arena);
+        S.cap = 0;
+        if (hipMalloc(&S.arena, need) != hipSuccess) {
+            (void)hipGetLastError();
+            S.arena = nullptr;
+            return false;
+        }
+        S.cap = need;
+    }
+    auto at = [&](size_t o) { return reinterpret_cast<double *>(S.arena + o); };
+    S.B.state = reinterpret_cast<psk::SpreadState *>(S.arena + state);
+    S.B.part = at(part);
+    S.B.alpha = at(alpha);
+    S.B.beta = at(beta);
+    S.B.area = at(area);
+    S.B.done = reinterpret_cast<int *>(S.arena + done);
+    S.jobs = reinterpret_cast<psk::SpreadJob *>(S.arena + jobs);
+    S.tasks = reinterpret_cast<psk::SpreadTask *>(S.arena + tasks);
+    return true;
+}
+
+// Runs the fits of jobs (all with or all without the Lambert column) on the stream; results to d_out.
+// Returns 1 when the buffers cannot be had and nothing has run (the caller then takes the other form).
+int spread_fits(Spread &S, hipStream_t stream, const std::vector<psk::SpreadJob> &all, const std::vector<int> &iters,
+                bool ls, int slots, size_t mfit, size_t nfac, ps_fit_result *d_out) {
+    constexpr int kCheck = 16;  // iterations launched between looks at the number of finished fits
+    for (size_t i0 = 0; i0 < all.size();) {
+        if (i0 > 0) HIPCHECK(hipStreamSynchronize(stream));  // the piece before still reads its tables
+        auto &jobs = S.hjobs;
+        jobs.clear();
+        int passes = 0, most = 0;
+        size_t i = i0;
+        for (; i < all.size() && (i == i0 || passes + all[i].npass <= kSpreadPasses); ++i) {
+            jobs.push_back(all[i]);
+            jobs.back().part0 = passes;
+            passes += all[i].npass;
+            most = std::max(most, iters[i]);
+        }
+        auto &tasks = S.htasks;
+        tasks = spread_tasks(jobs, slots);
+        if (!spread_buffers(S, jobs.size(), tasks.size(), passes, mfit, nfac)) {
+            if (i0 == 0) return 1;
+            return ps_fail(PS_ERR_NOMEM, "scratch allocation failed (%zu fits)", jobs.size());
+        }
+        HIPCHECK(hipMemcpyAsync(S.jobs, jobs.data(), sizeof(jobs[0]) * jobs.size(), hipMemcpyHostToDevice, stream));
+        HIPCHECK(hipMemcpyAsync(S.tasks, tasks.data(), sizeof(tasks[0]) * tasks.size(), hipMemcpyHostToDevice, stream));
+        const int nj = int(jobs.size());
+        hipLaunchKernelGGL(psk::spread_reset, dim3((nj + 255) / 256), dim3(256), 0, stream, S.B, nj);
+        hipLaunchKernelGGL(psk::spread_step, dim3(nj), dim3(psk::kWG2), 0, stream, S.jobs, S.B, d_out);
+        for (int it = 0; it <= most;) {  // the starting point and every iteration's trial point
+            for (int c = 0; c < kCheck && it <= most; ++c, ++it) {
+                if (ls)
+                    hipLaunchKernelGGL(psk::spread_eval<true>, dim3(tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs, S.tasks,
+                                       S.B, nullptr, nullptr, nullptr);
+                else
+                    hipLaunchKernelGGL(psk::spread_eval<false>, dim3(tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs, S.tasks,
+                                       S.B, nullptr, nullptr, nullptr);
+                hipLaunchKernelGGL(psk::spread_step, dim3(nj), dim3(psk::kWG2), 0, stream, S.jobs, S.B, d_out);
+            }
+            if (hipGetLastError() != hipSuccess) return ps_fail(PS_ERR_DEVICE, "spread fit launch failed");
+            if (it > most) break;
+            int done = 0;
+            HIPCHECK(hipMemcpyAsync(&done, S.B.done, sizeof(int), hipMemcpyDeviceToHost, stream));
+            HIPCHECK(hipStreamSynchronize(stream));
+            if (done == nj) break;
+        }
+        i0 = i;
+    }
+    return PS_OK;
+}
+
+psk::SpreadJob spread_job(const ps_handle *h, double freq, int pole, double conw_r, int out) {
+    return {h->dP2, freq, conw_r, pole, h->orbit, out, 0, h->P2.npass, 0};
+}
+int iteration_cap(const ps_handle *h) { return std::max({h->P.n_iter_max, h->P.n_iter_min, 0}); }
+
+// Up to this share of the resident workgroups, fits are spread: one workgroup each would leave so much of
+// the chip idle that two launches per iteration and the solves' latency cost less (figures: ps_spread.h).
+constexpr double kSpreadShare = 0.55;
+}  // namespace
+
 extern "C" int ps_set_precision(ps_handle *h, int precision) {
     if (!h) return ps_fail(PS_ERR_ARG, "ps_set_precision: null handle");
     if (precision != PS_FP64 && precision != PS_MIXED)
@@ -836,7 +989,8 @@ extern "C" int ps_get_info(const ps_handle *h, ps_info *info) {
 namespace {
 // Uploads one batch of fits of a problem and launches the fit kernel on the problem's stream, without
 // waiting: the results land in h->d_out.  Validation is the caller's.
-int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, double conw_r) {
+// spread: the fits beyond whole rounds of the resident workgroups may take the spread form.
+int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, double conw_r, bool spread) {
     if (nfits > h->cap_fits) {
         (void)hipFree(h->d_freq);
         (void)hipFree(h->d_pole);
@@ -851,15 +1005,38 @@ int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, d
         h->cap_fits = nfits;
     }
     int rc = set_conw(h, conw_r);
-    if (rc == PS_OK) rc = ensure_scratch(h, use_v2(h));
     if (rc != PS_OK) return rc;
+    // the last fits, short of a round
+    int rest = 0;
+    if (spread && use_v2(h) && h->orbit) {
+        rest = nfits % h->slots2;
+        if (rest > kSpreadShare * h->slots2) rest = 0;
+    }
+    int main = nfits - rest;
+    if (main > 0) {
+        rc = ensure_scratch(h, use_v2(h));
+        if (rc != PS_OK) return rc;
+    }
     HIPCHECK(hipMemcpyAsync(h->d_freq, freq, sizeof(double) * nfits, hipMemcpyHostToDevice, h->stream));
     HIPCHECK(hipMemcpyAsync(h->d_pole, pole, sizeof(int) * nfits, hipMemcpyHostToDevice, h->stream));
     HIPCHECK(hipEventRecord(h->ev0, h->stream));
-    if (use_v2(h)) {
-        const int grid = std::min(nfits, h->slots2);
+    if (rest > 0) {
+        std::vector<psk::SpreadJob> jobs(rest);
+        for (int i = 0; i < rest; ++i) jobs[i] = spread_job(h, freq[main + i], pole[main + i], conw_r, main + i);
+        rc = spread_fits(h->spread, h->stream, jobs, std::vector<int>(rest, iteration_cap(h)), h->ls, h->slots2, h->mfit,
+                         h->nfac, h->d_out);
+        if (rc < 0) return rc;
+        if (rc == 1) {
+            main = nfits;
+            rc = ensure_scratch(h, true);
+            if (rc != PS_OK) return rc;
+        }
+    }
+    if (main == 0) {
+    } else if (use_v2(h)) {
+        const int grid = std::min(main, h->slots2);
         rc = dispatch_model(h, [&]<class Model>() {
-            return h->ls ? launch_fit2<Model, true>(h, grid, nfits, conw_r) : launch_fit2<Model, false>(h, grid, nfits, conw_r);
+            return h->ls ? launch_fit2<Model, true>(h, grid, main, conw_r) : launch_fit2<Model, false>(h, grid, main, conw_r);
         });
     } else {
         const int grid = std::min(nfits, h->slots);
@@ -900,7 +1077,7 @@ extern "C" int ps_fit_batch(ps_handle *h, int nfits, const double *freq, const i
     if (rc != PS_OK) return rc;
     if (!(conw_r > 0)) return ps_fail(PS_ERR_ARG, "ps_fit_batch: conw_r must be positive");
     HIPCHECK(hipSetDevice(h->device));
-    rc = enqueue_fits(h, nfits, freq, pole, conw_r);
+    rc = enqueue_fits(h, nfits, freq, pole, conw_r, true);
     return rc != PS_OK ? rc : collect_fits(h, nfits, out);
 }
 
@@ -948,7 +1125,7 @@ extern "C" int ps_fit_multi(ps_handle *const *hs, int nh, const double *conw_r, 
             f[i].push_back(freq[j]);
             pl[i].push_back(pole[j]);
         }
-        rc = enqueue_fits(hs[i], int(jobs[i].size()), f[i].data(), pl[i].data(), conw_r[i]);
+        rc = enqueue_fits(hs[i], int(jobs[i].size()), f[i].data(), pl[i].data(), conw_r[i], false);
         if (rc != PS_OK) return rc;
     }
     std::vector<ps_fit_result> res;
@@ -1097,6 +1274,7 @@ extern "C" int ps_get_kernel(const ps_handle *h) {
 // ---------------------------------------------------------------------------------------------
 struct ps_batch {
     int device = 0;
+    Spread spread;
     std::vector<ps_handle *> hs;
     std::vector<double> cost;  // estimated work of one fit of each problem
     hipStream_t stream = nullptr;
@@ -1126,6 +1304,7 @@ extern "C" void ps_batch_release(ps_batch *b) {
     if (b->stream) hipStreamSynchronize(b->stream);
     if (b->exec) hipGraphExecDestroy(b->exec);
     for (void *p : b->owned) hipFree(p);
+    hipFree(b->spread.arena);
     hipFree(b->d_jobs);
     hipFree(b->d_out);
     if (b->ev0) hipEventDestroy(b->ev0);
@@ -1294,42 +1473,83 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
         HIPCHECK(hipMalloc(&b->d_out, sizeof(ps_fit_result) * njobs));
         b->cap_jobs = njobs;
     }
-    HIPCHECK(hipMemcpyAsync(b->d_conw, conw_r, sizeof(double) * nh, hipMemcpyHostToDevice, b->stream));
-    HIPCHECK(hipMemcpyAsync(b->d_jobs, jobs.data(), sizeof(psk::QueueJob) * njobs, hipMemcpyHostToDevice, b->stream));
-    if (!b->exec || b->exec_n0 != n0 || b->exec_n1 != n1) {
-        if (b->exec) hipGraphExecDestroy(b->exec);
-        b->exec = nullptr;
-        hipGraph_t g = nullptr;
-        HIPCHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        hipLaunchKernelGGL(psk::queue_reset, dim3(1), dim3(64), 0, b->stream, b->d_counter, 2);
-        if (b->mixed) {
-            if (n0)
-                hipLaunchKernelGGL(psk::queue_kernel_mixed<false>, dim3(std::min(n0, b->slots)), dim3(kWG), 0, b->stream,
-                                   b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs, n0, b->d_counter, b->d_out);
-            if (n1)
-                hipLaunchKernelGGL(psk::queue_kernel_mixed<true>, dim3(std::min(n1, b->slots)), dim3(kWG), 0, b->stream,
-                                   b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs + n0, n1, b->d_counter + 1,
-                                   b->d_out);
-        } else {
-            auto launch = [&](auto *kern, int njob, const psk::QueueJob *job, int *counter) {
-                if (njob)
-                    hipLaunchKernelGGL(kern, dim3(std::min(njob, b->slots)), dim3(psk::kWG2), 0, b->stream, b->d_probs,
-                                       b->d_layout, b->d_conw, b->pool, job, njob, counter, b->d_out);
-            };
-            launch(b->orbit ? psk::queue_kernel2<true, false> : psk::queue_kernel2<false, false>, n0, b->d_jobs, b->d_counter);
-            launch(b->orbit ? psk::queue_kernel2<true, true> : psk::queue_kernel2<false, true>, n1, b->d_jobs + n0,
-                   b->d_counter + 1);
+    // Few fits for the chip, or one that outlasts the rest: the spread form.  In passes of 288 facets: the
+    // queue ends no earlier than its longest fit and no earlier than the work shared out over the
+    // resident workgroups; the spread form shares it out evenly and pays for two launches and a solve
+    // per iteration (about three passes).
+    bool spread = false;
+    if (b->orbit) {
+        double sum = 0, longest = 0;
+        for (int j = 0; j < njobs; ++j) {
+            const ps_handle *h = b->hs[prob[j]];
+            const double w = double(h->P2.npass) * h->nfac / 288;
+            sum += w;
+            longest = std::max(longest, w);
         }
-        hipError_t e = hipStreamEndCapture(b->stream, &g);
-        if (e == hipSuccess) e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
-        if (g) hipGraphDestroy(g);
-        if (e != hipSuccess) return ps_fail(PS_ERR_DEVICE, "ps_batch_run: graph capture failed: %s", hipGetErrorString(e));
-        b->exec_n0 = n0;
-        b->exec_n1 = n1;
+        const double share = kSpreadPaired * sum / b->slots;
+        spread = share * 1.1 + 3 < std::max(longest, share + 0.5 * longest);
     }
-    HIPCHECK(hipEventRecord(b->ev0, b->stream));
-    HIPCHECK(hipGraphLaunch(b->exec, b->stream));
-    HIPCHECK(hipEventRecord(b->ev1, b->stream));
+    if (spread) {
+        size_t mfit = 1, nfac = 1;
+        for (const ps_handle *h : b->hs) {
+            mfit = std::max(mfit, size_t(h->mfit));
+            nfac = std::max(nfac, size_t(h->nfac));
+        }
+        HIPCHECK(hipEventRecord(b->ev0, b->stream));
+        for (int part = 0; part < 2 && spread; ++part) {
+            std::vector<psk::SpreadJob> sj;
+            std::vector<int> iters;
+            for (int k = part ? n0 : 0; k < (part ? njobs : n0); ++k) {
+                const ps_handle *h = b->hs[jobs[k].prob];
+                sj.push_back(spread_job(h, jobs[k].freq, jobs[k].pole, conw_r[jobs[k].prob], jobs[k].out));
+                iters.push_back(iteration_cap(h));
+            }
+            if (sj.empty()) continue;
+            if (part && n0) HIPCHECK(hipStreamSynchronize(b->stream));  // the first part's tables
+            rc = spread_fits(b->spread, b->stream, sj, iters, part == 1, b->slots, mfit, nfac, b->d_out);
+            if (rc < 0) return rc;
+            if (rc == 1) spread = false;  // no memory for it: the queue runs everything
+        }
+        if (spread) HIPCHECK(hipEventRecord(b->ev1, b->stream));
+    }
+    if (!spread) {
+        HIPCHECK(hipMemcpyAsync(b->d_conw, conw_r, sizeof(double) * nh, hipMemcpyHostToDevice, b->stream));
+        HIPCHECK(hipMemcpyAsync(b->d_jobs, jobs.data(), sizeof(psk::QueueJob) * njobs, hipMemcpyHostToDevice, b->stream));
+        if (!b->exec || b->exec_n0 != n0 || b->exec_n1 != n1) {
+            if (b->exec) hipGraphExecDestroy(b->exec);
+            b->exec = nullptr;
+            hipGraph_t g = nullptr;
+            HIPCHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+            hipLaunchKernelGGL(psk::queue_reset, dim3(1), dim3(64), 0, b->stream, b->d_counter, 2);
+            if (b->mixed) {
+                if (n0)
+                    hipLaunchKernelGGL(psk::queue_kernel_mixed<false>, dim3(std::min(n0, b->slots)), dim3(kWG), 0, b->stream,
+                                       b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs, n0, b->d_counter, b->d_out);
+                if (n1)
+                    hipLaunchKernelGGL(psk::queue_kernel_mixed<true>, dim3(std::min(n1, b->slots)), dim3(kWG), 0, b->stream,
+                                       b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs + n0, n1, b->d_counter + 1,
+                                       b->d_out);
+            } else {
+                auto launch = [&](auto *kern, int njob, const psk::QueueJob *job, int *counter) {
+                    if (njob)
+                        hipLaunchKernelGGL(kern, dim3(std::min(njob, b->slots)), dim3(psk::kWG2), 0, b->stream, b->d_probs,
+                                           b->d_layout, b->d_conw, b->pool, job, njob, counter, b->d_out);
+                };
+                launch(b->orbit ? psk::queue_kernel2<true, false> : psk::queue_kernel2<false, false>, n0, b->d_jobs, b->d_counter);
+                launch(b->orbit ? psk::queue_kernel2<true, true> : psk::queue_kernel2<false, true>, n1, b->d_jobs + n0,
+                       b->d_counter + 1);
+            }
+            hipError_t e = hipStreamEndCapture(b->stream, &g);
+            if (e == hipSuccess) e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
+            if (g) hipGraphDestroy(g);
+            if (e != hipSuccess) return ps_fail(PS_ERR_DEVICE, "ps_batch_run: graph capture failed: %s", hipGetErrorString(e));
+            b->exec_n0 = n0;
+            b->exec_n1 = n1;
+        }
+        HIPCHECK(hipEventRecord(b->ev0, b->stream));
+        HIPCHECK(hipGraphLaunch(b->exec, b->stream));
+        HIPCHECK(hipEventRecord(b->ev1, b->stream));
+    }
     HIPCHECK(hipMemcpyAsync(out, b->d_out, sizeof(ps_fit_result) * njobs, hipMemcpyDeviceToHost, b->stream));
     HIPCHECK(hipStreamSynchronize(b->stream));
     float ms = 0;
@@ -1378,8 +1598,25 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     if (!(conw_r > 0)) return ps_fail(PS_ERR_ARG, "ps_eval: conw_r must be positive");
     HIPCHECK(hipSetDevice(h->device));
     int rc = set_conw(h, conw_r);
-    if (rc == PS_OK) rc = ensure_scratch(h, use_v2(h));
     if (rc != PS_OK) return rc;
+    // few vectors: their passes spread over the chip
+    bool spread = use_v2(h) && h->orbit && h->P2.npass > 1 && nvec <= kSpreadShare * h->slots2 &&
+                  long(nvec) * h->P2.npass <= kSpreadPasses;
+    std::vector<psk::SpreadJob> sjobs;
+    std::vector<psk::SpreadTask> stasks;
+    if (spread) {
+        for (int v = 0; v < nvec; ++v) {
+            sjobs.push_back(spread_job(h, 0, 0, conw_r, v));
+            sjobs.back().part0 = v * h->P2.npass;
+        }
+        stasks = spread_tasks(sjobs, h->slots2);
+        spread = spread_buffers(h->spread, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac);
+    }
+    if (!spread) {
+        rc = ensure_scratch(h, use_v2(h));
+        if (rc != PS_OK) return rc;
+    }
+    const bool ls = h->ls || dyda;  // the Lambert columns are fitted or part of the raw rows
     const size_t mf2 = size_t(h->mfit) * h->mfit, nv = size_t(nvec);
     // staging buffers kept by the handle: allocated on first use, grown when a call needs more
     auto &E = h->ev;
@@ -1392,11 +1629,25 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     double *d_y = ymod ? E.y : nullptr, *d_dy = dyda ? E.dy : nullptr;
     HIPCHECK(hipMemcpyAsync(E.a, a, sizeof(double) * nv * h->ma, hipMemcpyHostToDevice, h->stream));
     HIPCHECK(hipEventRecord(h->ev0, h->stream));
-    if (use_v2(h)) {
+    if (spread) {
+        Spread &S = h->spread;
+        HIPCHECK(hipMemcpyAsync(S.jobs, sjobs.data(), sizeof(sjobs[0]) * sjobs.size(), hipMemcpyHostToDevice, h->stream));
+        HIPCHECK(hipMemcpyAsync(S.tasks, stasks.data(), sizeof(stasks[0]) * stasks.size(), hipMemcpyHostToDevice, h->stream));
+        auto launch = [&](auto *kern) {
+            hipLaunchKernelGGL(kern, dim3(stasks.size()), dim3(psk::kWG2), 0, h->stream, S.jobs, S.tasks, S.B,
+                               static_cast<const double *>(E.a), d_y, d_dy);
+        };
+        launch(ls ? psk::spread_eval<true> : psk::spread_eval<false>);
+        hipLaunchKernelGGL(psk::spread_sum, dim3(nvec), dim3(psk::kWG2), 0, h->stream, S.jobs, S.B, d_al, d_be, d_ch);
+        rc = hipGetLastError() == hipSuccess ? PS_OK : PS_ERR_DEVICE;
+    } else if (use_v2(h)) {
         const int grid = std::min(nvec, h->slots2);
         rc = dispatch_model(h, [&]<class Model>() {
-            hipLaunchKernelGGL((psk::eval_kernel2<Model, kMaxFac>), dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2,
-                               h->S2, E.a, nvec, conw_r, d_al, d_be, d_ch, d_y, d_dy);
+            auto launch = [&](auto *kern) {
+                hipLaunchKernelGGL(kern, dim3(grid), dim3(psk::kWG2), 0, h->stream, h->dP2, h->S2,
+                                   static_cast<const double *>(E.a), nvec, conw_r, d_al, d_be, d_ch, d_y, d_dy);
+            };
+            launch(ls ? psk::eval_kernel2<Model, true, kMaxFac> : psk::eval_kernel2<Model, false, kMaxFac>);
             return hipGetLastError() == hipSuccess ? PS_OK : PS_ERR_DEVICE;
         });
     } else {
@@ -1437,6 +1688,7 @@ extern "C" void ps_release(ps_handle *h) {
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     for (void *p : h->owned) hipFree(p);
+    hipFree(h->spread.arena);
     hipFree(h->d_freq);
     hipFree(h->d_pole);
     hipFree(h->d_out);

@@ -102,7 +102,7 @@ __device__ inline void curv_orbit(const DevProblem &P, const double *a, Shared2<
         t0[k] = t1[k] = 0;
         if (i < P.nf) {
             const double ar = gload(P.darea, i) * exp(facet_shape_sum(P, a, i));
-            area[i] = ar;
+            if (area) area[i] = ar;
             t0[k] = ar * cl;
             t1[k] = LS ? ar : ar * cls;
         }
@@ -858,6 +858,38 @@ __device__ __forceinline__ void stash_io(int nb, int ow, Prec<false>::V4 acc[kOw
 }
 
 // ---------------------------------------------------------------------------------------------
+// Pass k of an evaluation (phases B-D), after curv and the pole matrices: the Gram blocks of the pass's
+// rows alone into acc, those of the returned ownership set.  The caller adds the passes up in their
+// order, one sum after the other, wherever the passes run: a fit gets the same bits from one workgroup
+// that walks all passes and from passes spread over many (ps_spread.h).
+// ---------------------------------------------------------------------------------------------
+template <class Model, bool LS, int NFM>
+__device__ __forceinline__ int eval_pass(const DevProblem &P, Shared2<NFM> &sh, double wqc, int k, int nb,
+                                         const double *area, double *raw_y, double *raw_dyda,
+                                         Prec<false>::V4 acc[kOwn]) {
+    // the schedule through the scalar cache: wave-uniform trip counts and row ranges
+    const int tile0 = uload(P.pass_tile0, k), ntl = uload(P.pass_tile0, k + 1) - tile0;
+    const int u0 = uload(P.pass_unit0, k), u1 = uload(P.pass_unit0, k + 1);
+    // the facet loop issues at the lowest wave priority: when the other workgroup on the CU is in a
+    // latency-bound phase (lightcurve sums, Gram, Gauss-Jordan), its instructions go first and the
+    // facet loop fills the gaps
+    __builtin_amdgcn_s_setprio(0);
+    Model::template rows<LS>(P, sh, tile0, ntl, k, k == P.npass - 1, area, raw_y, raw_dyda);
+    __builtin_amdgcn_s_setprio(2);
+    const PassRowData rd = load_pass_rows(P, tile0, wqc);
+    __syncthreads();
+    normalise_pass(P, sh, rd, u0, u1);
+    __syncthreads();
+    // The ownership sets with three blocks go to waves 0, 1 in even passes and 2, 3 in odd ones, so the
+    // Gram work falls evenly on the four SIMDs
+    const int ow = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + 2 * (k & 1)) & 3;
+#pragma unroll
+    for (int b = 0; b < kOwn; ++b) acc[b] = Prec<false>::zero();
+    gram_pass(nb, P, sh, rd, ntl, ow, acc);
+    return ow;
+}
+
+// ---------------------------------------------------------------------------------------------
 // mrqcof for the parameters in sh.a: alpha[mfit][mfit], beta[mfit] to the given buffers, chi2
 // returned.  raw_y / raw_dyda: the raw rows (ps_eval).
 // ---------------------------------------------------------------------------------------------
@@ -865,37 +897,24 @@ template <class Model, bool LS, int NFM>
 __device__ __forceinline__ double mrqcof2(const DevProblem &P, Shared2<NFM> &sh, double wqc, double *area,
                                           double *stash, double *alpha, double *beta, double *raw_y,
                                           double *raw_dyda) {
-    using Pd = Prec<false>;
     Model::template curv<LS>(P, sh.a, sh, area);
     blmatrix_lds(sh.a[P.nc], sh.a[P.nc + 1], sh);
     __syncthreads();
     const int npass = P.npass;
     const int nb = (P.mfit + 16) >> 4;  // 16-column blocks covering mfit + 1 columns
     for (int k = 0; k < npass; ++k) {
-        // the schedule through the scalar cache: wave-uniform trip counts and row ranges
-        const int tile0 = uload(P.pass_tile0, k), ntl = uload(P.pass_tile0, k + 1) - tile0;
-        const int u0 = uload(P.pass_unit0, k), u1 = uload(P.pass_unit0, k + 1);
-        const bool last = k == npass - 1;
-        // the facet loop issues at the lowest wave priority: when the other workgroup on the CU is in a
-        // latency-bound phase (lightcurve sums, Gram, Gauss-Jordan), its instructions go first and the
-        // facet loop fills the gaps
-        __builtin_amdgcn_s_setprio(0);
-        Model::template rows<LS>(P, sh, tile0, ntl, k, last, area, raw_y, raw_dyda);
-        __builtin_amdgcn_s_setprio(2);
-        const PassRowData rd = load_pass_rows(P, tile0, wqc);
-        __syncthreads();
-        normalise_pass(P, sh, rd, u0, u1);
-        __syncthreads();
-        // the accumulators live only through phase D: parked in the slot between passes.  The
-        // ownership sets with three blocks go to waves 0, 1 in even passes and 2, 3 in odd ones, so the
-        // Gram work falls evenly on the four SIMDs
-        const int ow = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + 2 * (k & 1)) & 3;
-        Pd::V4 acc[kOwn];
+        Prec<false>::V4 acc[kOwn];
+        const int ow = eval_pass<Model, LS>(P, sh, wqc, k, nb, area, raw_y, raw_dyda, acc);
+        // the sum of the passes lives in the slot: the facet loop needs the registers
+        if (k > 0) {
+            Prec<false>::V4 sum[kOwn];
 #pragma unroll
-        for (int b = 0; b < kOwn; ++b) acc[b] = Pd::zero();
-        if (k > 0) stash_io(nb, ow, acc, stash, false);
-        gram_pass(nb, P, sh, rd, ntl, ow, acc);
-        if (last)
+            for (int b = 0; b < kOwn; ++b) sum[b] = Prec<false>::zero();
+            stash_io(nb, ow, sum, stash, false);
+#pragma unroll
+            for (int b = 0; b < kOwn; ++b) acc[b] = sum[b] + acc[b];
+        }
+        if (k == npass - 1)
             gram_store(nb, P, sh, ow, acc, alpha, beta);
         else
             stash_io(nb, ow, acc, stash, true);
@@ -1028,56 +1047,34 @@ __device__ inline SlotPtrs slot_ptrs(const Slots2 &S, int slot) {
     return p;
 }
 
-template <class Model, bool LS, int NFM>
-__device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, const SlotPtrs &sp, double freq,
-                                        int pole, double conw_r, ps_fit_result *out) {
-    const int tid = threadIdx.x;
-    const int nc = P.nc, ma = P.ma, mfit = P.mfit;
-    double *const area = sp.area;
-    const double wqc = conv_weight(conw_r);
-    if (pole < 1 || pole > PS_N_POLES || !(freq > 0) || !(conw_r > 0)) {
-        // a job the host did not check (ps_fit_batch_noalloc reads device arrays): no fit, niter = -1
-        if (tid == 0) {
-            const double nan = __builtin_nan("");
-            *out = {nan, nan, nan, nan, nan, nan, nan, -1, 0};
-        }
-        __syncthreads();
-        return;
-    }
-    // initial parameters (:819-844)
-    if (tid < ma) {
-        double v;
-        const int m = pole - 1;
-        if (tid < nc)
-            v = P.cg_first[tid];
-        else if (tid == nc)
-            v = P.pole_beta[m];
-        else if (tid == nc + 1)
-            v = P.pole_lambda[m];
-        else if (tid == nc + 2)
-            v = 24 * 2 * kPi / (1 / freq);
-        else if (tid < nc + 6)
-            v = (tid == nc + 3) ? P.par1 : (tid == nc + 4) ? P.par2 : P.par3;
-        else if (tid == nc + 6)
-            v = P.log_cl;
-        else
-            v = 1;
-        sh.cg[tid] = v;
-    }
-    __syncthreads();
-    int cur = 0;
+// A job the host did not check (ps_fit_batch_noalloc reads device arrays): no fit, niter = -1.
+__device__ inline bool job_valid(double freq, int pole, double conw_r) {
+    return pole >= 1 && pole <= PS_N_POLES && freq > 0 && conw_r > 0;
+}
+
+// The initial parameter tid of a fit (period_search_BOINC.cpp:819-844).
+__device__ inline double initial_param(const DevProblem &P, int tid, double freq, int pole) {
+    const int nc = P.nc, m = pole - 1;
+    if (tid < nc) return P.cg_first[tid];
+    if (tid == nc) return P.pole_beta[m];
+    if (tid == nc + 1) return P.pole_lambda[m];
+    if (tid == nc + 2) return 24 * 2 * kPi / (1 / freq);
+    if (tid < nc + 6) return (tid == nc + 3) ? P.par1 : (tid == nc + 4) ? P.par2 : P.par3;
+    return tid == nc + 6 ? P.log_cl : 1;
+}
+
+// The state of the LM loop (mrqmin.c with the driver's bookkeeping).  It is wave-uniform.  The compiler
+// cannot see that: its values meet at the joins of lane-predicated stores (tid < ma), so settle()
+// re-asserts them after each such region; the loop exit and the accept / reject decisions then branch
+// on scalars.
+struct LmState {
     double alamda = -1, ochisq = 0, chisq = 0, rchisq = -1;
     double iter_diff = 1e40, dev_old = 1e30, dev_new = 0;
     double chck0 = 0, chck1 = 0, chck2 = 0;
     int niter = 0, nfail = 0;
-    // the LM controls and state are wave-uniform.  The compiler cannot see that for the state: its
-    // values meet at the joins of lane-predicated stores (tid < ma), so settle() re-asserts them after
-    // each such region; the loop exit and the accept / reject decisions then branch on scalars.
-    const int n_iter_max = __builtin_amdgcn_readfirstlane(P.n_iter_max);
-    const int n_iter_min = __builtin_amdgcn_readfirstlane(P.n_iter_min);
-    const double iter_diff_max = uniform_double(P.iter_diff_max), alamda_start = uniform_double(P.alamda_start);
-    const double alamda_incr = uniform_double(P.alamda_incr);
-    auto settle = [&] {
+    int cur = 0;  // the buffer of the accepted normal equations
+    int err = 0;  // the last solve's status
+    __device__ void settle() {
         alamda = uniform_double(alamda);
         ochisq = uniform_double(ochisq);
         chisq = uniform_double(chisq);
@@ -1091,77 +1088,150 @@ __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, c
         niter = __builtin_amdgcn_readfirstlane(niter);
         nfail = __builtin_amdgcn_readfirstlane(nfail);
         cur = __builtin_amdgcn_readfirstlane(cur);
-    };
+        err = __builtin_amdgcn_readfirstlane(err);
+    }
+    // the driver's stop rule (period_search_BOINC.cpp:868-872)
+    __device__ bool more(const DevProblem &P) const {
+        return ((niter < __builtin_amdgcn_readfirstlane(P.n_iter_max)) && (iter_diff > uniform_double(P.iter_diff_max))) ||
+               (niter < __builtin_amdgcn_readfirstlane(P.n_iter_min));
+    }
+    // the starting point has been evaluated (mrqmin.c:34-52)
+    __device__ void start(double chi) {
+        ochisq = chi;
+        chisq = chi;  // a failed first step then reports this fit's own starting chi2
+    }
+    // a trial point has been evaluated (mrqmin.c:80-107): true if it is accepted
+    __device__ bool judge(double chi, const DevProblem &P) {
+        const double incr = uniform_double(P.alamda_incr);
+        chisq = chi;
+        if (chisq < ochisq) {
+            alamda = alamda / incr;
+            cur ^= 1;
+            return true;
+        }
+        alamda = incr * alamda;
+        chisq = ochisq;
+        return false;
+    }
+    // after an iteration: the rms and its improvement (period_search_BOINC.cpp:884-893)
+    __device__ void rms(const DevProblem &P) {
+        dev_new = sqrt(rchisq / __builtin_amdgcn_readfirstlane(P.nobs));
+        if (dev_old - dev_new > 1e-10) {
+            iter_diff = dev_old - dev_new;
+            dev_old = dev_new;
+        }
+    }
+    __device__ void convexity(const double s[3], double conw_r) {
+        chck0 = s[0];
+        chck1 = s[1];
+        chck2 = s[2];
+        rchisq = chisq - (chck0 * chck0 + chck1 * chck1 + chck2 * chck2) * (conw_r * conw_r);
+    }
+    __device__ ps_fit_result result(const double *cg, int nc, double totarea) const {
+        ps_fit_result r;
+        r.dev = dev_new;
+        r.prd = 2 * kPi / cg[nc + 2];
+        r.dark = sqrt(chck0 * chck0 + chck1 * chck1 + chck2 * chck2);
+        r.totarea = totarea;
+        r.la = (180 / kPi) * cg[nc + 1];
+        r.be = 90 - (180 / kPi) * cg[nc];
+        r.chisq = chisq;
+        r.niter = niter;
+        r.nsolve_fail = nfail;
+        return r;
+    }
+};
+
+// Solves the damped system of the accepted normal equations; on success the trial point (accepted
+// parameters plus the step, mrqmin.c:53-79) is in sh.atry and sh.a.  Returns gauss_jordan2's status.  A
+// failed solve changes nothing (mrqmin.c:61-63), so the next one, of the same matrix, fails alike: it is
+// not run again.
+template <int NFM>
+__device__ __forceinline__ int lm_solve(const DevProblem &P, Shared2<NFM> &sh, const LmState &lm, const double *al,
+                                        const double *be) {
+    if (lm.err != 0) return lm.err;
+    const int tid = threadIdx.x, mfit = P.mfit;
+    // the damped matrix: four reads in flight per lane; diagonal entries are every (mfit + 1)-th
+    const int nn = mfit * mfit;
+    for (int i0 = tid; i0 < nn; i0 += 4 * kWG2) {
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = i0 + u * kWG2 < nn ? al[i0 + u * kWG2] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int it = i0 + u * kWG2;
+            if (it < nn) sh.u.g.cov[it] = (it % (mfit + 1) == 0) ? v[u] * (1 + lm.alamda) : v[u];
+        }
+    }
+    for (int j = tid; j < mfit; j += kWG2) sh.da[j] = be[j];
+    __syncthreads();
+    const int err = __builtin_amdgcn_readfirstlane(gauss_jordan2(sh, mfit));
+    __syncthreads();
+    if (err == 0) {
+        if (tid < mfit) {
+            const int l = P.fit_idx[tid];
+            sh.atry[l] = sh.cg[l] + sh.da[tid];
+        }
+        __syncthreads();
+        if (tid < P.ma) sh.a[tid] = sh.atry[tid];
+    }
+    return err;
+}
+
+template <class Model, bool LS, int NFM>
+__device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, const SlotPtrs &sp, double freq,
+                                        int pole, double conw_r, ps_fit_result *out) {
+    const int tid = threadIdx.x;
+    const int ma = P.ma;
+    double *const area = sp.area;
+    const double wqc = conv_weight(conw_r);
+    if (!job_valid(freq, pole, conw_r)) {
+        if (tid == 0) {
+            const double nan = __builtin_nan("");
+            *out = {nan, nan, nan, nan, nan, nan, nan, -1, 0};
+        }
+        __syncthreads();
+        return;
+    }
+    if (tid < ma) sh.cg[tid] = initial_param(P, tid, freq, pole);
+    __syncthreads();
+    LmState lm;
     for (;;) {
-        settle();
-        if (!(((niter < n_iter_max) && (iter_diff > iter_diff_max)) || (niter < n_iter_min))) break;
+        lm.settle();
+        if (!lm.more(P)) break;
         // One mrqcof per pass: the first pass evaluates the starting point (mrqmin.c:34-52), later
         // passes solve the damped system and evaluate the trial point (mrqmin.c:53-79).
-        const bool init = alamda < 0;
-        int err = 0;
+        const bool init = lm.alamda < 0;
         bool fresh = false;  // the step was accepted: cg is the trial point just evaluated
         if (init) {
-            alamda = alamda_start;
+            lm.alamda = uniform_double(P.alamda_start);
             if (tid < ma) sh.a[tid] = sh.cg[tid];
         } else {
-            // the damped matrix: four reads in flight per lane; diagonal entries are every (mfit + 1)-th
-            const double *al = cur ? sp.alpha1 : sp.alpha0;
-            const int nn = mfit * mfit;
-            for (int i0 = tid; i0 < nn; i0 += 4 * kWG2) {
-                double v[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = i0 + u * kWG2 < nn ? al[i0 + u * kWG2] : 0.0;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int it = i0 + u * kWG2;
-                    if (it < nn) sh.u.g.cov[it] = (it % (mfit + 1) == 0) ? v[u] * (1 + alamda) : v[u];
-                }
-            }
-            for (int j = tid; j < mfit; j += kWG2) sh.da[j] = (cur ? sp.beta1 : sp.beta0)[j];
-            __syncthreads();
-            err = __builtin_amdgcn_readfirstlane(gauss_jordan2(sh, mfit));
-            __syncthreads();
-            if (err == 0) {
-                if (tid < mfit) {
-                    const int l = P.fit_idx[tid];
-                    sh.atry[l] = sh.cg[l] + sh.da[tid];
-                }
-                __syncthreads();
-                if (tid < ma) sh.a[tid] = sh.atry[tid];
-            }
+            lm.err = lm_solve(P, sh, lm, lm.cur ? sp.alpha1 : sp.alpha0, lm.cur ? sp.beta1 : sp.beta0);
         }
-        if (err == 0) {
+        if (lm.err == 0) {
             __syncthreads();
             // the starting point fills the current buffers, a trial point the other ones
             const bool other = !init;
             const double chi = uniform_double(mrqcof2<Model, LS>(P, sh, wqc, area, sp.stash,
-                                                                 (cur ^ other) ? sp.alpha1 : sp.alpha0,
-                                                                 (cur ^ other) ? sp.beta1 : sp.beta0, nullptr, nullptr));
+                                                                 (lm.cur ^ other) ? sp.alpha1 : sp.alpha0,
+                                                                 (lm.cur ^ other) ? sp.beta1 : sp.beta0, nullptr, nullptr));
             if (init) {
-                ochisq = chi;
-                chisq = chi;  // a failed first step then reports this fit's own starting chi2
+                lm.start(chi);
                 if (tid < ma) sh.atry[tid] = sh.cg[tid];
-            } else {
-                chisq = chi;
-                if (chisq < ochisq) {
-                    alamda = alamda / alamda_incr;
-                    cur ^= 1;
-                    fresh = true;
-                    if (tid < ma) sh.cg[tid] = sh.atry[tid];
-                } else {
-                    alamda = alamda_incr * alamda;
-                    chisq = ochisq;
-                }
+            } else if (lm.judge(chi, P)) {
+                fresh = true;
+                if (tid < ma) sh.cg[tid] = sh.atry[tid];
             }
             __syncthreads();
         } else {
-            ++nfail;
+            ++lm.nfail;
         }
-        settle();
+        lm.settle();
         if (init) continue;
-        ++niter;
-        if (niter == 1 || chisq < ochisq) {
-            ochisq = chisq;
+        ++lm.niter;
+        if (lm.niter == 1 || lm.chisq < lm.ochisq) {
+            lm.ochisq = lm.chisq;
             if (tid < ma) sh.a[tid] = sh.cg[tid];
             __syncthreads();
             // curv(cg) (period_search_BOINC.cpp:874); after an accepted step cg is the trial point, whose
@@ -1178,34 +1248,16 @@ __device__ __forceinline__ void fit_one(const DevProblem &P, Shared2<NFM> &sh, c
                 }
             }
             __syncthreads();
-            chck0 = uniform_double(sh.scal[1]);
-            chck1 = uniform_double(sh.scal[2]);
-            chck2 = uniform_double(sh.scal[3]);
-            rchisq = chisq - (chck0 * chck0 + chck1 * chck1 + chck2 * chck2) * (conw_r * conw_r);
+            const double sn[3] = {uniform_double(sh.scal[1]), uniform_double(sh.scal[2]), uniform_double(sh.scal[3])};
+            lm.convexity(sn, conw_r);
             __syncthreads();
         }
-        settle();
-        dev_new = sqrt(rchisq / __builtin_amdgcn_readfirstlane(P.nobs));
-        if (dev_old - dev_new > 1e-10) {
-            iter_diff = dev_old - dev_new;
-            dev_old = dev_new;
-        }
+        lm.settle();
+        lm.rms(P);
     }
     if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
         const double totarea = facet_sum(area, nullptr, P.nf);
-        if (tid == 0) {
-            ps_fit_result r;
-            r.dev = dev_new;
-            r.prd = 2 * kPi / sh.cg[nc + 2];
-            r.dark = sqrt(chck0 * chck0 + chck1 * chck1 + chck2 * chck2);
-            r.totarea = totarea;
-            r.la = (180 / kPi) * sh.cg[nc + 1];
-            r.be = 90 - (180 / kPi) * sh.cg[nc];
-            r.chisq = chisq;
-            r.niter = niter;
-            r.nsolve_fail = nfail;
-            *out = r;
-        }
+        if (tid == 0) *out = lm.result(sh.cg, P.nc, totarea);
     }
     __syncthreads();
 }
@@ -1336,8 +1388,9 @@ __global__ void queue_reset(int *counter, int n) {
     if (int(threadIdx.x) < n) counter[threadIdx.x] = 0;
 }
 
-// mrqcof for externally supplied parameter vectors (ps_eval), J-free.
-template <class Model, int NFM>
+// mrqcof for externally supplied parameter vectors (ps_eval), J-free.  LS: the Lambert columns are fitted
+// or asked for (raw rows).
+template <class Model, bool LS, int NFM>
 __global__ __launch_bounds__(kWG2, 2) void eval_kernel2(const DevProblem *__restrict__ Pp, Slots2 S, const double *avec,
                                                      int nvec, double conw_r, double *alpha, double *beta,
                                                      double *chisq, double *raw_y, double *raw_dyda) {
@@ -1351,7 +1404,7 @@ __global__ __launch_bounds__(kWG2, 2) void eval_kernel2(const DevProblem *__rest
     for (int v = blockIdx.x; v < nvec; v += gridDim.x) {
         if (tid < P.ma) sh.a[tid] = avec[size_t(v) * P.ma + tid];
         __syncthreads();
-        const double c = mrqcof2<Model, true>(P, sh, conv_weight(conw_r), area, stash, al, be,
+        const double c = mrqcof2<Model, LS>(P, sh, conv_weight(conw_r), area, stash, al, be,
                                                   raw_y ? raw_y + size_t(v) * P.npts : nullptr,
                                                   raw_dyda ? raw_dyda + size_t(v) * P.npts * P.ma : nullptr);
         for (int it = tid; it < mfit * mfit; it += kWG2)
