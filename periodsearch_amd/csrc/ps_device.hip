@@ -698,7 +698,11 @@ extern "C" int ps_prepare(const ps_input *in, const ps_geometry *geo, int device
         const int nsched = int(sc.perm.size()), nq = nsched + psk::kPassRows;
         std::vector<double> qt(nq, 0), qex(nq, 0), qey(nq, 0), qez(nq, 0), qsx(nq, 0), qsy(nq, 0), qsz(nq, 0),
             qal(nq, 0), qy(nq, 0), qsig(nq, 1), qsl(nq, 0);
-        std::vector<int> qrel(nq, 0), qperm(nq, -1);
+        std::vector<int> qrel(nq, 0), qperm(nq, -1), qunit(nq, -1);
+        for (int k = 0; k + 1 < int(sc.pass_tile0.size()); ++k)
+            for (int u = sc.pass_unit0[k]; u < sc.pass_unit0[k + 1]; ++u)
+                for (int r = sc.unit_rows[u] & 255; r < sc.unit_rows[u] >> 8; ++r)
+                    qunit[16 * sc.pass_tile0[k] + r] = u - sc.pass_unit0[k];
         h->wq2_host.assign(nq, 0.0);
         for (int q = 0; q < nsched; ++q) {
             const int p = sc.perm[q];
@@ -743,6 +747,7 @@ extern "C" int ps_prepare(const ps_input *in, const ps_geometry *geo, int device
         Q.unit_rows = dev_upload(sc.unit_rows.data(), sc.unit_rows.size(), o);
         Q.unit_lc = dev_upload(sc.unit_lc.data(), sc.unit_lc.size(), o);
         Q.qrel = dev_upload(qrel.data(), nq, o);
+        Q.qunit = dev_upload(qunit.data(), nq, o);
         Q.qperm = dev_upload(qperm.data(), nq, o);
         Q.fpos = dev_upload(fpos.data(), fpos.size(), o);
         Q.qsl = dev_upload(qsl.data(), nq, o);

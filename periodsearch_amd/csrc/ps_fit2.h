@@ -34,6 +34,7 @@ constexpr int kPassRows = 16 * kPassTiles;
 constexpr int kJP = 57;                       // LDS row pitch (doubles): mfit + 1 <= 57 for Lmax <= 6
 constexpr int kGJRows2 = (kMaxFit + kWaves2 - 1) / kWaves2;  // Gauss-Jordan rows per wave
 constexpr int kOwn = 3;                       // Gram blocks owned per wave
+constexpr int kUnitSums = 2;                  // lightcurves summed between two barriers of phase C
 constexpr int kCholP = 65;                    // row pitch of the Cholesky factor (odd: lane = row without bank conflicts)
 
 template <int NFM>
@@ -50,7 +51,7 @@ struct Shared2 {
     };
     union {
         double da[64];       // the LM step: the Gauss-Jordan right-hand side, then its solution
-        double csum[2][64];  // phase C: the column sums of two consecutive lightcurves
+        double csum[kUnitSums][64];  // phase C: the column sums of the lightcurves between two barriers
     };
     double bl[9], hbl[18];  // pole rotation, the pole-frame generators of its derivatives
     double scal[4];
@@ -617,20 +618,22 @@ struct OrbitModel {
     }
 };
 
-// Per-row data of a pass for phases C and D, loaded once after phase B (the loads overlap the barrier):
-// lane i holds pass rows i and 64 + i.  y: the observation, sl: sig*Lpoints of a relative point
-// (coef = sl/ave, mrqcof.c:94), w: the weight w/sig^2.
+// Per-row data of a pass for phases C and D, loaded once after phase B (the loads overlap the barrier).
+// Phase C: lane l of the two waves of group g holds row 64g + l, y: the observation, sl: sig*Lpoints of a
+// relative point (coef = sl/ave, mrqcof.c:94), unit: its lightcurve among the pass's (-1: calibrated or
+// padding).  Phase D: the weights w/sig^2 of rows l and 64 + l.
 struct PassRowData {
-    double y_a, y_b, sl_a, sl_b, w_a, w_b;
+    double y, sl, w_a, w_b;
+    int unit;
 };
 // wqc: the weight of the three convexity rows, 1/sig^2 with sig = 1/conw_r (period_search_BOINC.cpp:721-726),
 // formed by the kernel from the call's conw_r.
 __device__ inline PassRowData load_pass_rows(const DevProblem &P, int tile0, double wqc) {
-    const int c = threadIdx.x & 63;
+    const int c = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);
     const int q = tile0 * 16 + c;  // the point arrays are padded by a whole pass
     const bool ca = q >= P.conv_q && q < P.conv_q + 3, cb = q + 64 >= P.conv_q && q + 64 < P.conv_q + 3;
-    return {gload(P.y, q), gload(P.y, q + 64), gload(P.qsl, q), gload(P.qsl, q + 64), ca ? wqc : gload(P.wq, q),
-            cb ? wqc : gload(P.wq, q + 64)};
+    return {gload(P.y, q + 64 * g), gload(P.qsl, q + 64 * g), ca ? wqc : gload(P.wq, q), cb ? wqc : gload(P.wq, q + 64),
+            gload(P.qunit, q + 64 * g)};
 }
 __device__ inline double conv_weight(double conw_r) {
     const double sig = 1 / conw_r;
@@ -643,75 +646,68 @@ __device__ inline double conv_weight(double conw_r) {
 // coef = sig*Lpoints/ave; dyda_c <- coef*(dyda_c - (ymod*dave_c)*(1/ave)), the c00 column 0, and the
 // residual column y - coef*ymod.  The column sums are split over the waves: lane (pl, kg) of wave w
 // adds column 16w + pl over the rows r0 + kg, r0 + kg + 4, ..., the four row classes are added across
-// the lane groups in a fixed order, ((0 + 1) + (2 + 3)), and the 64 sums go through LDS (sh.csum, two
-// units in flight, so one barrier per unit suffices).  Each wave then normalises rows r0 + w, r0 + w + 4, ... with lane c
-// on column c, taking the per-row factors from lane i (pass rows i and 64 + i).
+// the lane groups in a fixed order, ((0 + 1) + (2 + 3)).  The sums of two units go to LDS, then,
+// after one barrier, lane = row: each of the two waves of a row group takes half of the columns, with the
+// row's factors in its registers and its unit's sums read from LDS (a broadcast for all rows of a unit).
+// With lane = column and a barrier per unit, the factors came through four lane reads a row and the
+// divisions stood in every unit's chain: 9700 cycles of a pass of two units (2560 fits of 6 iterations at 2400
+// points and 288 facets 27.0 ms, now 26.0).
 // ---------------------------------------------------------------------------------------------
 template <int NFM>
 __device__ inline void normalise_pass(const DevProblem &P, Shared2<NFM> &sh, const PassRowData &rd, int u0, int u1) {
     const int c = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pl = c & 15, kg = c >> 4;
-    const int mfit = P.mfit, c00col = P.c00col;
+    const int mfit = P.mfit;
     const int *unit_rows = P.unit_rows;
-    // the columns the row loop writes: the residual and c00 columns are written separately
-    const bool wcol = c < mfit && c != c00col;
-    const int cl = min(c, mfit);  // the column a lane reads (lanes past mfit read a valid one, unused)
     // the summed column, clamped: lanes past mfit add a valid column and their sums are not used
     const int scol = min(16 * wave + pl, mfit);
-    const double ym_a = sh.u.rows[c * kJP + mfit], ym_b = sh.u.rows[(64 + c) * kJP + mfit];
-    for (int u = u0; u < u1; ++u) {
-        const int rg = uload(unit_rows, u), r0 = rg & 255, r1 = rg >> 8;
-        // class kg: rows r0 + kg, r0 + kg + 4, ... of the whole groups of four, in order; the rows past
-        // the last whole group go to class 0, in order
-        const int nfull = (r1 - r0) >> 2;
-        const double *cp = sh.u.rows + (r0 + kg) * kJP + scol;  // the lane's class, row by row
-        double sk = 0;
-        int i = 0;
-        for (; i + 4 <= nfull; i += 4) {  // four reads in flight, added in row order
-            double x[4];
+    const int half = wave & 1, mid = (mfit + 1) >> 1;
+    double *row = sh.u.rows + (64 * (wave >> 1) + c) * kJP;
+    const double ym = row[mfit];
+    for (int ub = u0; ub < u1; ub += kUnitSums) {
+        const int ue = min(u1, ub + kUnitSums);
+        for (int u = ub; u < ue; ++u) {
+            const int rg = uload(unit_rows, u), r0 = rg & 255, r1 = rg >> 8;
+            // class kg: rows r0 + kg, r0 + kg + 4, ... of the whole groups of four, in order; the rows past
+            // the last whole group go to class 0, in order
+            const int nfull = (r1 - r0) >> 2;
+            const double *cp = sh.u.rows + (r0 + kg) * kJP + scol;  // the lane's class, row by row
+            double sk = 0;
+            int i = 0;
+            for (; i + 4 <= nfull; i += 4) {  // four reads in flight, added in row order
+                double x[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) x[j] = cp[(4 * (i + j)) * kJP];
+                for (int j = 0; j < 4; ++j) x[j] = cp[(4 * (i + j)) * kJP];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) sk += x[j];
-        }
-        for (; i < nfull; ++i) sk += cp[(4 * i) * kJP];
-        for (int r = r0 + 4 * nfull; r < r1; ++r) {
-            const double x = sh.u.rows[r * kJP + scol];
-            sk += kg == 0 ? x : 0.0;
-        }
-        double *cs = sh.csum[(u - u0) & 1];
-        const double sw = sum_groups(sk);  // (class 0 + class 1) + (class 2 + class 3)
-        if (kg == 0) cs[16 * wave + pl] = sw;
-        // every wave has read the rows of the unit and written its sums
-        __syncthreads();
-        const double s = cs[c], ave = cs[mfit];
-        const double rave = 1 / ave;
-        const double coef_a = rd.sl_a / ave, coef_b = rd.sl_b / ave;
-        const double res_a = rd.y_a - coef_a * ym_a, res_b = rd.y_b - coef_b * ym_b;
-        // The residual column and the c00 column (0) of row r: by lane r (or r - 64) of the wave that
-        // normalises the row, so that every row is written by one wave.
-        auto fixed_cols = [&](int r, double res) {
-            if (r >= r0 && r < r1 && (r - r0) % kWaves2 == wave) {
-                double *row = sh.u.rows + r * kJP;
-                row[mfit] = res;
-                if (c00col >= 0) row[c00col] = 0.0;
+                for (int j = 0; j < 4; ++j) sk += x[j];
             }
-        };
-        fixed_cols(c, res_a);
-        fixed_cols(64 + c, res_b);
-        // the other columns of row r, with the row's factors from lane r (rows below 64) or r - 64: the
-        // two halves as two loops, so the lane reads need no selects
-        auto update = [&](int r, double coef, double ym) {
-            double *row = sh.u.rows + r * kJP;
-            const double v = coef * (row[cl] - (ym * s) * rave);
-            if (wcol) row[c] = v;
-        };
-        int r = r0 + wave;
-        const int rm = min(r1, 64);
+            for (; i < nfull; ++i) sk += cp[(4 * i) * kJP];
+            for (int r = r0 + 4 * nfull; r < r1; ++r) {
+                const double x = sh.u.rows[r * kJP + scol];
+                sk += kg == 0 ? x : 0.0;
+            }
+            const double sw = sum_groups(sk);  // (class 0 + class 1) + (class 2 + class 3)
+            if (kg == 0) sh.csum[u - ub][16 * wave + pl] = sw;
+        }
+        // every wave has read the rows of the units and written its sums
+        __syncthreads();
+        const int uu = rd.unit - (ub - u0);
+        if (rd.unit >= 0 && uu >= 0 && uu < ue - ub) {
+            const double *s = sh.csum[uu];
+            const double ave = s[mfit];
+            const double rave = 1 / ave, coef = rd.sl / ave;
+            const int j0 = half ? mid : P.c00col + 1, j1 = half ? mfit : mid;  // c00 is column 0 where it is fitted
 #pragma unroll 4
-        for (; r < rm; r += kWaves2) update(r, read_lane(coef_a, r), read_lane(ym_a, r));
-#pragma unroll 4
-        for (; r < r1; r += kWaves2) update(r, read_lane(coef_b, r - 64), read_lane(ym_b, r - 64));
+            for (int j = j0; j < j1; ++j) {
+                const double v = coef * (row[j] - (ym * s[j]) * rave);
+                row[j] = v;
+            }
+            if (half)
+                row[mfit] = rd.y - coef * ym;
+            else if (P.c00col >= 0)
+                row[0] = 0.0;
+        }
+        if (ue < u1) __syncthreads();  // the sums are read before the next units' overwrite them
     }
 }
 

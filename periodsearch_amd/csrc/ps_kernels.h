@@ -78,6 +78,7 @@ struct DevProblem {
     int npass, nsched, conv_q, c00col;
     const int *pass_tile0, *pass_unit0, *unit_rows, *unit_lc;
     const int *qrel;   // [nsched] 1: the position holds a point of a relative lightcurve
+    const int *qunit;  // [nsched] the point's lightcurve among its pass's units (-1: calibrated, padding)
     const int *qperm;  // [nsched] the point's index in input order (-1: padding)
     const int *fpos;   // [ma] the row column of a parameter (-1: fixed); column mfit = the residual
     const double *qsl; // [nsched] sig*Lpoints of a relative lightcurve's point (mrqcof.c:94), else 0
