@@ -35,7 +35,6 @@ constexpr int kJP = 57;                       // LDS row pitch (doubles): mfit +
 constexpr int kGJRows2 = (kMaxFit + kWaves2 - 1) / kWaves2;  // Gauss-Jordan rows per wave
 constexpr int kOwn = 3;                       // Gram blocks owned per wave
 constexpr int kUnitSums = 2;                  // lightcurves summed between two barriers of phase C
-constexpr int kCholP = 65;                    // row pitch of the Cholesky factor (odd: lane = row without bank conflicts)
 
 template <int NFM>
 struct Shared2 {
@@ -1144,95 +1143,6 @@ struct LmState {
     }
 };
 
-// ---------------------------------------------------------------------------------------------
-// The damped system by L D L^T, one wave: the matrix sh.u.c.m (lower triangle, row n = the right-hand
-// side) is symmetric and, damped, positive definite, so it needs no pivoting (a full search would only
-// ever find diagonal elements).  Panels of 16 columns: the blocks left of the panel are subtracted on
-// v_mfma_f64_16x16x4f64, then lane i carries row i through the panel's columns in registers, the pivot
-// row's entries as scalars from v_readlane; row n becomes D^-1 L^-1 b on the way.  Back substitution
-// leaves x_k in lane k.  Returns false, with nothing decided, when a pivot is not a normal positive number
-// (not positive definite to rounding, a column of rounding noise or overflow, NaN): the caller then runs
-// gauss_errc's elimination, which has the reference's answer to such systems.
-//
-// What bounds it: the chain of one column (read a lane, reciprocal, scale, update: about 100 cycles), 55
-// times.  The elimination it stands for takes 55 workgroup barriers and a pivot search over the whole
-// matrix.  Measured, 6 iterations at 2400 points and 288 facets: one step of 10 fits (sum, solve,
-// bookkeeping) 90 -> 30 us, the 10 fits 1.16 -> 0.67 ms, 2560 fits 29.3 -> 27.0 ms.
-// ---------------------------------------------------------------------------------------------
-__device__ inline void wave_lds_fence() {  // LDS written by the wave's lanes before, read by others after
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-template <int NFM>
-__device__ __forceinline__ bool cholesky_solve(Shared2<NFM> &sh, int n, double &x) {
-    using Pd = Prec<false>;
-    constexpr double kLeast = 1e-270, kMost = 1e270;
-    const int lane = threadIdx.x & 63, pl = lane & 15, kg = lane >> 4;
-    double *m = sh.u.c.m, *d = sh.u.c.d;
-    const int nrb = (n + 16) >> 4;  // row blocks, the right-hand side's row included
-    for (int kb = 0; 16 * kb < n; ++kb) {
-        if (kb > 0) {
-            Pd::V4 acc[3];
-#pragma unroll
-            for (int t = 0; t < 3; ++t) acc[t] = Pd::zero();
-            const double *mb = m + (16 * kb + pl) * kCholP + kg;
-            for (int s = 0; s < 4 * kb; ++s) {
-                const double bv = mb[4 * s] * d[4 * s + kg];
-                double av[3];
-#pragma unroll
-                for (int t = 0; t < 3; ++t) av[t] = kb + t < nrb ? mb[(16 * t) * kCholP + 4 * s] : 0.0;
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    if (kb + t < nrb) acc[t] = Pd::mma(av[t], bv, acc[t]);
-            }
-#pragma unroll
-            for (int t = 0; t < 3; ++t)
-                if (kb + t < nrb)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) m[(16 * (kb + t) + Pd::row(r, kg)) * kCholP + 16 * kb + pl] -= acc[t][r];
-            wave_lds_fence();
-        }
-        double p[16], dv = 0;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) p[c] = m[lane * kCholP + 16 * kb + c];
-        const int left = n - 16 * kb;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            if (j < left) {
-                const double dj = read_lane(p[j], 16 * kb + j);
-                if (!(dj > kLeast && dj < kMost)) return false;
-                dv = pl == j ? dj : dv;
-                double r = __builtin_amdgcn_rcp(dj);
-                const double e = fma(-dj, r, 1.0);
-                r = fma(r, fma(e, e, e), r);  // third order, as in orbit_loop
-                const double l = p[j] * r;
-#pragma unroll
-                for (int c = j + 1; c < 16; ++c) p[c] = fma(-l, read_lane(p[j], 16 * kb + c), p[c]);
-                p[j] = l;
-            }
-        }
-        if (lane >= 16 * kb) {
-#pragma unroll
-            for (int c = 0; c < 16; ++c) m[lane * kCholP + 16 * kb + c] = p[c];
-        }
-        if (kg == 0) d[16 * kb + pl] = dv;
-        wave_lds_fence();
-    }
-    // x_j, last first: lane k takes L[j][k] x_j from its sum
-    x = lane < n ? m[n * kCholP + lane] : 0.0;
-    for (int j0 = n - 1; j0 >= 0; j0 -= 8) {
-        double lr[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) lr[u] = m[max(j0 - u, 0) * kCholP + lane];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int j = j0 - u;
-            if (j > 0) x = fma(lane < j ? -lr[u] : 0.0, read_lane(x, j), x);
-        }
-    }
-    return true;
-}
-
 // Solves the damped system of the accepted normal equations; on success the trial point (accepted
 // parameters plus the step, mrqmin.c:53-79) is in sh.atry and sh.a.  Returns gauss_jordan2's status.  A
 // failed solve changes nothing (mrqmin.c:61-63), so the next one, of the same matrix, fails alike: it is
@@ -1241,35 +1151,9 @@ template <int NFM>
 __device__ __forceinline__ int lm_solve(const DevProblem &P, Shared2<NFM> &sh, const LmState &lm, const double *al,
                                         const double *be) {
     if (lm.err != 0) return lm.err;
-    const int tid = threadIdx.x, mfit = P.mfit, l = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    {
-        // lane = column, the waves take the rows in turn, all of a wave's reads in flight
-        constexpr int kRows = (kMaxFit + kWaves2 - 1) / kWaves2;
-        double v[kRows], vb = 0;
-#pragma unroll
-        for (int k = 0; k < kRows; ++k) {
-            const int r = wave + kWaves2 * k;
-            v[k] = (r < mfit && l < mfit) ? al[r * mfit + l] : 0.0;
-        }
-        if (wave == 0 && l < mfit) vb = be[l];
-#pragma unroll
-        for (int k = 0; k < kRows; ++k) {
-            const int r = wave + kWaves2 * k;
-            if (r < mfit) sh.u.c.m[r * kCholP + l] = l == r ? v[k] * (1 + lm.alamda) : v[k];
-        }
-        if (wave == 0) sh.u.c.m[mfit * kCholP + l] = vb;
-    }
-    __syncthreads();
-    if (wave == 0) {
-        double x = 0;
-        const bool ok = cholesky_solve(sh, mfit, x);
-        if (l < mfit) sh.da[l] = x;
-        if (l == 0) sh.u.c.ok = ok;
-    }
-    __syncthreads();
+    const int tid = threadIdx.x, mfit = P.mfit;
     int err = 0;
-    if (!__builtin_amdgcn_readfirstlane(sh.u.c.ok)) {
+    if (!cholesky_step<kWaves2>(sh, mfit, lm.alamda, al, be)) {
         __syncthreads();
         // the damped matrix again, four reads in flight per lane; diagonal entries are every (mfit + 1)-th
         const int nn = mfit * mfit;

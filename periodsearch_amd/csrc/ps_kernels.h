@@ -38,6 +38,7 @@ constexpr int kRes = kMap - 1;  // J column holding the residual after phase C (
 constexpr int kMaxFac = 512;    // nrows <= 8
 constexpr int kTP = 2;          // 16-point tiles per wave per pass of the facet loop
 constexpr int kDsphLds = 288 * 49;  // FP64 Dsph held in LDS (facets x pitch: nrows <= 6, Lmax <= 6), else read from L2
+constexpr int kCholP = 65;      // row pitch of the Cholesky factor (odd: lane = row without bank conflicts)
 constexpr double kTiny = 1e-8;  // period_search/constants.h:10
 constexpr double kPi = M_PI;
 
@@ -124,6 +125,11 @@ struct Shared {
             double red_v[2][kWaves];     // each wave's candidate |a| and index
             int red_q[2][kWaves];
         } g;
+        struct {
+            double m[64 * kCholP];   // Cholesky: the damped matrix with the right-hand side as one more row, then L
+            double d[64];
+            int ok;
+        } c;
         struct {
             double red[64 * 64];     // phase D: cross-wave sum of the normal equations
         } d;
@@ -989,6 +995,129 @@ __device__ inline double read_lane(double x, int l) {  // x of lane l (l wave-un
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
+// ---------------------------------------------------------------------------------------------
+// The damped system by L D L^T, one wave: the matrix m (lower triangle, row n = the right-hand
+// side) is symmetric and, damped, positive definite, so it needs no pivoting (a full search would only
+// ever find diagonal elements).  Panels of 16 columns: the blocks left of the panel are subtracted on
+// v_mfma_f64_16x16x4f64, then lane i carries row i through the panel's columns in registers, the pivot
+// row's entries as scalars from v_readlane; row n becomes D^-1 L^-1 b on the way.  Back substitution
+// leaves x_k in lane k.  Returns false, with nothing decided, when a pivot is not a normal positive number
+// (not positive definite to rounding, a column of rounding noise or overflow, NaN): the caller then runs
+// gauss_errc's elimination, which has the reference's answer to such systems.
+//
+// What bounds it: the chain of one column (read a lane, reciprocal, scale, update: about 100 cycles), 55
+// times.  The elimination it stands for takes 55 workgroup barriers and a pivot search over the whole
+// matrix.  Measured, 6 iterations at 2400 points and 288 facets: one step of 10 fits (sum, solve,
+// bookkeeping) 90 -> 30 us, the 10 fits 1.16 -> 0.67 ms, 2560 fits 29.3 -> 27.0 ms; in the FP64
+// materialised-Jacobian kernels 310 fits of 1 - 2 thousand points in curves of up to 400 9.9 -> 9.1 ms.
+// ---------------------------------------------------------------------------------------------
+__device__ inline void wave_lds_fence() {  // LDS written by the wave's lanes before, read by others after
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bool cholesky_solve(double *m, double *d, int n, double &x) {
+    using Pd = Prec<false>;
+    constexpr double kLeast = 1e-270, kMost = 1e270;
+    const int lane = threadIdx.x & 63, pl = lane & 15, kg = lane >> 4;
+    const int nrb = (n + 16) >> 4;  // row blocks, the right-hand side's row included
+    for (int kb = 0; 16 * kb < n; ++kb) {
+        if (kb > 0) {
+            Pd::V4 acc[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) acc[t] = Pd::zero();
+            const double *mb = m + (16 * kb + pl) * kCholP + kg;
+            for (int s = 0; s < 4 * kb; ++s) {
+                const double bv = mb[4 * s] * d[4 * s + kg];
+                double av[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t) av[t] = kb + t < nrb ? mb[(16 * t) * kCholP + 4 * s] : 0.0;
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    if (kb + t < nrb) acc[t] = Pd::mma(av[t], bv, acc[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+                if (kb + t < nrb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) m[(16 * (kb + t) + Pd::row(r, kg)) * kCholP + 16 * kb + pl] -= acc[t][r];
+            wave_lds_fence();
+        }
+        double p[16], dv = 0;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) p[c] = m[lane * kCholP + 16 * kb + c];
+        const int left = n - 16 * kb;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            if (j < left) {
+                const double dj = read_lane(p[j], 16 * kb + j);
+                if (!(dj > kLeast && dj < kMost)) return false;
+                dv = pl == j ? dj : dv;
+                double r = __builtin_amdgcn_rcp(dj);
+                const double e = fma(-dj, r, 1.0);
+                r = fma(r, fma(e, e, e), r);  // third order: v_rcp_f64 is good to 2^-24
+                const double l = p[j] * r;
+#pragma unroll
+                for (int c = j + 1; c < 16; ++c) p[c] = fma(-l, read_lane(p[j], 16 * kb + c), p[c]);
+                p[j] = l;
+            }
+        }
+        if (lane >= 16 * kb) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) m[lane * kCholP + 16 * kb + c] = p[c];
+        }
+        if (kg == 0) d[16 * kb + pl] = dv;
+        wave_lds_fence();
+    }
+    // x_j, last first: lane k takes L[j][k] x_j from its sum
+    x = lane < n ? m[n * kCholP + lane] : 0.0;
+    for (int j0 = n - 1; j0 >= 0; j0 -= 8) {
+        double lr[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) lr[u] = m[max(j0 - u, 0) * kCholP + lane];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int j = j0 - u;
+            if (j > 0) x = fma(lane < j ? -lr[u] : 0.0, read_lane(x, j), x);
+        }
+    }
+    return true;
+}
+
+// The damped system of the normal equations al, be into sh.u.c and its solution into sh.da, by all waves of
+// a workgroup of WAVES (the first one solves).  False: cholesky_solve declined.
+template <int WAVES, class SH>
+__device__ __forceinline__ bool cholesky_step(SH &sh, int n, double alamda, const double *al, const double *be) {
+    const int l = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    {
+        // lane = column, the waves take the rows in turn, all of a wave's reads in flight
+        constexpr int kRows = (kMaxFit + WAVES - 1) / WAVES;
+        double v[kRows], vb = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+            const int r = wave + WAVES * k;
+            v[k] = (r < n && l < n) ? al[r * n + l] : 0.0;
+        }
+        if (wave == 0 && l < n) vb = be[l];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+            const int r = wave + WAVES * k;
+            if (r < n) sh.u.c.m[r * kCholP + l] = l == r ? v[k] * (1 + alamda) : v[k];
+        }
+        if (wave == 0) sh.u.c.m[n * kCholP + l] = vb;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        double x = 0;
+        const bool ok = cholesky_solve(sh.u.c.m, sh.u.c.d, n, x);
+        if (l < n) sh.da[l] = x;
+        if (l == 0) sh.u.c.ok = ok;
+    }
+    __syncthreads();
+    const bool ok = __builtin_amdgcn_readfirstlane(sh.u.c.ok);
+    __syncthreads();
+    return ok;
+}
+
 constexpr int kGJRows = (kMaxFit + kWaves - 1) / kWaves;  // rows held per wave
 
 __device__ inline int gauss_jordan(Shared &sh, int n) {
@@ -1211,20 +1340,26 @@ __device__ __forceinline__ void fit_one_legacy(const DevProblem &P, Shared &sh, 
             alamda = P.alamda_start;
             if (tid < ma) sh.a[tid] = sh.cg[tid];
         } else {
-            for (int it = tid; it < mfit * mfit; it += kWG) {
-                const int j = it / mfit, k = it - j * mfit;
-                const double v = (cur ? alpha1 : alpha0)[it];
-                const double d = (j == k) ? v * (1 + alamda) : v;
-                sh.u.g.cov[it] = d;
-                if (MIX) sh.u.g.cov0[it] = d;
+            // FP64: Cholesky, the elimination where it declines; mixed precision refines with the inverse the
+            // elimination leaves
+            bool solved = false;
+            if constexpr (!MIX) solved = cholesky_step<kWaves>(sh, mfit, alamda, cur ? alpha1 : alpha0, cur ? beta1 : beta0);
+            if (!solved) {
+                for (int it = tid; it < mfit * mfit; it += kWG) {
+                    const int j = it / mfit, k = it - j * mfit;
+                    const double v = (cur ? alpha1 : alpha0)[it];
+                    const double d = (j == k) ? v * (1 + alamda) : v;
+                    sh.u.g.cov[it] = d;
+                    if (MIX) sh.u.g.cov0[it] = d;
+                }
+                for (int j = tid; j < mfit; j += kWG) {
+                    sh.da[j] = (cur ? beta1 : beta0)[j];
+                    if (MIX) sh.b0[j] = sh.da[j];
+                }
+                __syncthreads();
+                err = __builtin_amdgcn_readfirstlane(gauss_jordan(sh, mfit));
+                __syncthreads();
             }
-            for (int j = tid; j < mfit; j += kWG) {
-                sh.da[j] = (cur ? beta1 : beta0)[j];
-                if (MIX) sh.b0[j] = sh.da[j];
-            }
-            __syncthreads();
-            err = __builtin_amdgcn_readfirstlane(gauss_jordan(sh, mfit));
-            __syncthreads();
             if (MIX && err == 0) refine_solution(sh, mfit);
             if (err == 0) {
                 if (tid < mfit) {
