@@ -1487,18 +1487,26 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     // Few fits for the chip, or one that outlasts the rest: the spread form.  In passes of 288 facets: the
     // queue ends no earlier than its longest fit and no earlier than the work shared out over the
     // resident workgroups; the spread form shares it out evenly and pays for two launches and a solve
-    // per iteration (about three passes).
+    // per iteration (about three passes) of each piece that fits its buffers.  A piece lasts as long as
+    // its slowest fit, while a workgroup of the queue goes on to the next job: where fits may stop early
+    // (10 to 100 iterations, mean 33) 10240 fits of 512 asteroids in 44 pieces took 2073 ms spread
+    // against 746 ms queued, so then only what fits one piece is spread.
     bool spread = false;
     if (b->orbit) {
         double sum = 0, longest = 0;
+        long passes = 0;
+        bool early = false;
         for (int j = 0; j < njobs; ++j) {
             const ps_handle *h = b->hs[prob[j]];
+            passes += h->P2.npass;
+            early |= h->P.iter_diff_max > 0;
             const double w = double(h->P2.npass) * h->nfac / 288;
             sum += w;
             longest = std::max(longest, w);
         }
         const double share = kSpreadPaired * sum / b->slots;
-        spread = share * 1.1 + 3 < std::max(longest, share + 0.5 * longest);
+        const long pieces = (passes + kSpreadPasses - 1) / kSpreadPasses;
+        spread = share * 1.1 + 3 * pieces < std::max(longest, share + 0.5 * longest) && (!early || pieces == 1);
     }
     if (spread) {
         size_t mfit = 1, nfac = 1;
