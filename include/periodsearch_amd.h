@@ -158,7 +158,7 @@ int ps_fit_batch(ps_handle *h, int nfits, const double *freq, const int *pole, d
 /* The fits of several prepared problems (asteroids) on one device as one batch: job j fits frequency
    freq[j] (1/h) with pole pole[j] (1..10) of problem hs[prob[j]] at convexity weight
    conw_r[prob[j]], into out[j].  When every problem runs the FP64 J-free kernels this is
-   ps_batch_create + ps_batch_run + ps_batch_release (one persistent launch); otherwise each problem's
+   ps_batch_create + ps_batch_run + ps_batch_release; otherwise each problem's
    jobs run as one launch on its own stream, all issued (largest problem first) before any result is
    waited for.  Results equal ps_fit_batch's for the same fits.  Each problem handle may appear once.
    The per-job body is that of period_search_BOINC.cpp:817-921. */
@@ -184,9 +184,11 @@ int ps_fit_batch_noalloc(ps_handle *h, int nfits, const double *freq, const int 
    PS_ERR_ARG (precisions differ).  The handles must outlive the batch.
    ps_batch_run: njobs fits (job j: problem prob[j], frequency freq[j] in 1/h, pole pole[j] in 1..10, at
    convexity weight conw_r[prob[j]]) as one graph launch: a queue reset, then persistent workgroups
-   that claim jobs from a device work queue, longest first, until it is empty.  out[j] equals
-   ps_fit_batch's result for the same fit.  The graph is kept and replayed while the job counts repeat.
-   ps_batch_kernel_time: device time of the graph launches since the last reset (HIP events). */
+   that claim jobs from a device work queue, longest first, until it is empty.  FP64 batches with little
+   work for the chip, or with a fit that outlasts the rest, run as two launches per iteration over the
+   passes of all fits instead.  out[j] equals ps_fit_batch's result for the same fit.  The graph is
+   kept and replayed while the job counts repeat.
+   ps_batch_kernel_time: device time of the batch's launches since the last reset (HIP events). */
 typedef struct ps_batch ps_batch;
 int ps_batch_create(ps_handle *const *hs, int nh, ps_batch **out);
 int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const int *prob, const double *freq, const int *pole,
@@ -204,7 +206,8 @@ int ps_scan(ps_handle *h, int n_from, int n_to, double conw_r, ps_line *lines);
    (normalised normal equations, fitted parameters only); when ymod/dyda are non-NULL also the raw
    bright()/conv() outputs per point, ymod[nvec*npts], dyda[nvec*npts*ma], before lightcurve
    normalisation.  Any output pointer may be NULL.  The device staging is kept by the handle between
-   calls (grown when a call needs more).  The kernel time counts in ps_kernel_time. */
+   calls (grown when a call needs more); long lists are computed in chunks, whose outputs leave while
+   the next one is computed.  The kernel time counts in ps_kernel_time. */
 int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, double *alpha, double *beta, double *chisq,
             double *ymod, double *dyda);
 /* Device time of the fit and evaluation kernels since the last reset, measured with HIP events on the

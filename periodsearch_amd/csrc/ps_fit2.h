@@ -2,7 +2,7 @@
 // ps_kernels.h.
 //
 // One 256-lane workgroup (4 wave64) owns one (period, pole) fit, and two such workgroups share a CU
-// (LDS <= 80 KB and 256 VGPRs each): while one waits in the Gauss-Jordan pivot chain or at a
+// (LDS <= 80 KB and 256 VGPRs each): while one waits in the solve's pivot chain or at a
 // barrier, the other's facet loop issues.
 //
 // The Jacobian is never written to memory.  An evaluation (mrqcof, period_search/mrqcof.c:16-148)
@@ -49,7 +49,7 @@ struct Shared2 {
         orb_d2 tab[NFM + 8];             // orbit form: (Area*cl, Area*cls) by orbit, then eight zeros
     };
     union {
-        double da[64];       // the LM step: the Gauss-Jordan right-hand side, then its solution
+        double da[64];       // the LM step: the solve's right-hand side, then its solution
         double csum[kUnitSums][64];  // phase C: the column sums of the lightcurves between two barriers
     };
     double bl[9], hbl[18];  // pole rotation, the pole-frame generators of its derivatives
