@@ -22,6 +22,8 @@
 // After the last pass the blocks are alpha (J^T W J), beta (J^T W r) and chi2.
 #pragma once
 
+#include <cstddef>
+
 #include "ps_kernels.h"
 #include "ps_orbit.h"
 
@@ -56,7 +58,8 @@ struct Shared2 {
     double scal[4];
     double ascale, amax[kWaves2];  // orbit form: the power of two the table is scaled by, each wave's largest entry
     int job;  // the queue kernel: the job claimed by the workgroup
-    union {
+    // the orbit form's buffers of X lie in the rows and are read and written 16 bytes at a time
+    alignas(16) union {
         double rows[kPassRows * kJP];  // the pass's Jacobian rows (fitted columns + residual)
         struct {
             double cov[64 * 64];             // Gauss-Jordan: the damped matrix
@@ -71,6 +74,9 @@ struct Shared2 {
         } c;
     } u;
 };
+static_assert(offsetof(Shared2<kMaxFac>, u) % 16 == 0 && 64 * kJP * sizeof(double) % 16 == 0 && kXBytes % 16 == 0,
+              "every buffer of X starts on 16 bytes");
+static_assert(sizeof(Shared2<kMaxFac>) <= 80 * 1024, "two workgroups share a CU's 160 KB of LDS");
 
 // Per-slot device buffers of the J-free kernels.
 struct Slots2 {
