@@ -256,6 +256,7 @@ __device__ __forceinline__ void orbit_correct(const orb_u4 *corr, int norb, int 
     const int lane = threadIdx.x & 63, hi = lane >> 5, lo = lane & 31;
     // an odd orbit at the end: zeros beside it (the table has a zero orbit past the last one)
     if (cnt & 1) *reinterpret_cast<orb_u4 *>(xw + cnt * 1024 + lane * 16) = orb_u4{0, 0, 0, 0};
+    wave_lds_fence();  // X of all lanes, before any lane reads another's
     const char *xr = xw + hi * 1024 + lo * 16;
 #pragma unroll
     for (int t = 0; t < orb_ctiles(L); ++t) {
@@ -281,6 +282,7 @@ __device__ __forceinline__ void orbit_correct(const orb_u4 *corr, int norb, int 
             if (j + 4 < N) A.c[j + 4] += double(__uint_as_float(sw[1]));
         }
     }
+    wave_lds_fence();  // the next piece's X overwrites what other lanes have read here
 }
 
 }  // namespace psk

@@ -33,3 +33,34 @@ static_assert((rows + 64 * psk::kJP * sizeof(double)) % 16 == 0 && psk::kXBytes 
 static_assert(offsetof(psk::Shared2<psk::kMaxFac>, tab) % 16 == 0);
 static_assert(2 * sizeof(psk::Shared2<psk::kMaxFac>) <= 160 * 1024);
 """, "--cuda-host-only", "-fsyntax-only")
+
+
+def fences_around_lds(ir, kernel):
+    """The LDS accesses of a kernel's IR in order: 'w', 'r' and 'F' for a wavefront fence."""
+    body = ir[ir.index(f"@{kernel}("):]
+    body = body[:body.index("\n}")]
+    seq = []
+    for line in body.split("\n"):
+        if 'fence syncscope("wavefront' in line:
+            seq.append("F")
+        elif re.search(r"\bstore <4 x i32>", line) and "addrspace(3)" in line:
+            seq.append("w")
+        elif re.search(r"\bload <8 x bfloat>", line) and "addrspace(3)" in line:
+            seq.append("r")
+    return "".join(seq)
+
+
+def test_x_is_fenced_between_lanes(tmp_path):
+    """A lane reads the X of other lanes of its wave: a fence lies between the stores and the loads, and between
+    the loads and the next piece's stores."""
+    out = compile_probe(tmp_path, """
+extern "C" __global__ void probe(const psk::orb_u4 *corr, int norb, int cnt, double *res) {
+    __shared__ __attribute__((aligned(16))) char x[psk::kXBytes];
+    psk::OrbAcc<3, false> A;
+    A.clear();
+    psk::orbit_correct<3, false>(corr, norb, 0, cnt, x, A);
+    for (int j = 0; j < 16; ++j) res[16 * threadIdx.x + j] = A.c[j];
+}
+""", "--cuda-device-only", "-O1", "-S", "-emit-llvm")
+    seq = fences_around_lds(out.read_text(), "probe")
+    assert re.fullmatch(r"w+Fr+F", seq), seq
