@@ -469,13 +469,17 @@ __device__ __forceinline__ void model_rows2(const DevProblem &P, Shared2<NFM> &s
     }
 }
 
+// Whether a row belongs to a pass of ntl tiles (its last point group may run past it).
+__device__ constexpr bool pass_row(int row, int ntl) { return row < 16 * ntl; }
+
 // ---------------------------------------------------------------------------------------------
 // Phase B of one pass by symmetry orbits (ps_orbit.h): lane l of the two waves of group g owns pass row
 // 64g + l.  Each of the two sums its half of the orbits; they exchange through the row's own LDS
-// columns (once neither needs its buffer of X there any more): the first hands over its odd-l sums, the second its even-l sums and the six rotation sums,
-// and after a barrier the first completes the even-l columns and everything else of the row, the
-// second the odd-l columns.  The roles alternate with the pass, so that the longer epilogue falls on
-// every SIMD in turn.  A group with no row in the pass only joins the barrier.
+// columns (once neither needs its buffer of X there any more): the first hands over its odd-l sums, the
+// second its even-l sums and the six rotation sums, and after a barrier the first completes the even-l
+// columns and everything else of the row, the second the odd-l columns.  The roles alternate with the
+// pass, so that the longer epilogue falls on every SIMD in turn.  A group with no row in the pass only
+// joins the barrier.
 // ---------------------------------------------------------------------------------------------
 template <int L, bool LS, int NFM>
 __device__ __forceinline__ void model_rows_orbit(const DevProblem &P, Shared2<NFM> &sh, int tile0, int ntl, int turn,
@@ -536,7 +540,8 @@ __device__ __forceinline__ void model_rows_orbit(const DevProblem &P, Shared2<NF
         double dphp[3];
         const double asc = sh.ascale, phs = phase_scale(a, nc, al, eph, p1 * eph * al / (p2 * p2), dphp);
         const double scale = phs * asc;
-        const int orig = raw_dyda ? gload(P.qperm, q) : -1;
+        // the last group's lanes past the pass hold points of the next one, whose own lanes write their raw rows
+        const int orig = raw_dyda && pass_row(64 * g + lane, ntl) ? gload(P.qperm, q) : -1;
         double *rraw = raw_dyda + size_t(orig >= 0 ? orig : 0) * ma;
         auto shape = [&](int j) {  // a coefficient's column, complete
             const int col = uload(P.scol, j);
@@ -625,20 +630,20 @@ struct OrbitModel {
 
 // Per-row data of a pass for phases C and D, loaded once after phase B (the loads overlap the barrier).
 // Phase C: lane l of the two waves of group g holds row 64g + l, y: the observation, sl: sig*Lpoints of a
-// relative point (coef = sl/ave, mrqcof.c:94), unit: its lightcurve among the pass's (-1: calibrated or
-// padding).  Phase D: the weights w/sig^2 of rows l and 64 + l.
+// relative point (coef = sl/ave, mrqcof.c:94), unit: its lightcurve among the pass's (-1: calibrated,
+// padding or past the pass's ntl tiles).  Phase D: the weights w/sig^2 of rows l and 64 + l.
 struct PassRowData {
     double y, sl, w_a, w_b;
     int unit;
 };
 // wqc: the weight of the three convexity rows, 1/sig^2 with sig = 1/conw_r (period_search_BOINC.cpp:721-726),
 // formed by the kernel from the call's conw_r.
-__device__ inline PassRowData load_pass_rows(const DevProblem &P, int tile0, double wqc) {
+__device__ inline PassRowData load_pass_rows(const DevProblem &P, int tile0, int ntl, double wqc) {
     const int c = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);
     const int q = tile0 * 16 + c;  // the point arrays are padded by a whole pass
     const bool ca = q >= P.conv_q && q < P.conv_q + 3, cb = q + 64 >= P.conv_q && q + 64 < P.conv_q + 3;
     return {gload(P.y, q + 64 * g), gload(P.qsl, q + 64 * g), ca ? wqc : gload(P.wq, q), cb ? wqc : gload(P.wq, q + 64),
-            gload(P.qunit, q + 64 * g)};
+            pass_row(64 * g + c, ntl) ? gload(P.qunit, q + 64 * g) : -1};
 }
 __device__ inline double conv_weight(double conw_r) {
     const double sig = 1 / conw_r;
@@ -883,7 +888,7 @@ __device__ __forceinline__ int eval_pass(const DevProblem &P, Shared2<NFM> &sh, 
     __builtin_amdgcn_s_setprio(0);
     Model::template rows<LS>(P, sh, tile0, ntl, k, k == P.npass - 1, area, raw_y, raw_dyda);
     __builtin_amdgcn_s_setprio(2);
-    const PassRowData rd = load_pass_rows(P, tile0, wqc);
+    const PassRowData rd = load_pass_rows(P, tile0, ntl, wqc);
     __syncthreads();
     normalise_pass(P, sh, rd, u0, u1);
     __syncthreads();
