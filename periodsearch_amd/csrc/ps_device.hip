@@ -1297,14 +1297,13 @@ struct ps_batch {
     int *d_counter = nullptr;
     Slots2 pool{};
     bool mixed = false;  // mixed precision: queue_kernel_mixed over the legacy problem descriptions
-    bool orbit = false;  // every problem has symmetry orbits: queue_kernel2<true, .>
     Slots lpool{};       // its per-slot buffers
     int slots = 0;
     psk::QueueJob *d_jobs = nullptr;
     ps_fit_result *d_out = nullptr;
     int cap_jobs = 0;
     hipGraphExec_t exec = nullptr;
-    int exec_n0 = -1, exec_n1 = -1;
+    std::array<int, 5> exec_key{};  // the graph's first job and the job count of each of its kernels
     double kernel_ms = 0;
     int launches = 0;
 };
@@ -1357,12 +1356,10 @@ extern "C" int ps_batch_create(ps_handle *const *hs, int nh, ps_batch **out) {
     std::vector<int> layout(nh);
     size_t amax = 1, bmax = 1, fmax = 1, nptmax = 1, segmax = 1;
     b->cost.resize(nh);
-    b->orbit = !mixed;
-    for (int i = 0; i < nh; ++i) b->orbit = b->orbit && hs[i]->orbit != 0;
     for (int i = 0; i < nh; ++i) {
         const ps_handle *h = hs[i];
         probs[i] = mixed ? h->dP : h->dP2;
-        layout[i] = b->orbit ? h->orbit : layout_id(h->var);
+        layout[i] = !mixed && h->orbit ? h->orbit : layout_id(h->var);
         amax = std::max(amax, size_t(h->mfit) * h->mfit);
         bmax = std::max(bmax, size_t(h->mfit));
         fmax = std::max(fmax, size_t(h->nfac));
@@ -1377,8 +1374,8 @@ extern "C" int ps_batch_create(ps_handle *const *hs, int nh, ps_batch **out) {
     b->d_layout = dev_upload(layout.data(), nh, o);
     std::vector<double> zero(nh, 0.0);
     b->d_conw = dev_upload(zero.data(), nh, o);
-    int z2[2] = {0, 0};
-    b->d_counter = dev_upload(z2, 2, o);
+    const int z4[4] = {0, 0, 0, 0};
+    b->d_counter = dev_upload(z4, 4, o);
     for (void *p : o)
         if (!p) return fail(ps_fail(PS_ERR_DEVICE, "device upload failed"));
     hipDeviceProp_t prop;
@@ -1456,22 +1453,28 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
         if (changed)
             for (int i = 0; i < nh; ++i) HIPCHECK(hipStreamSynchronize(b->hs[i]->stream));
     }
-    // the job queue: problems without the Lambert column first, then those with it; each group longest first
+    // The job queue in four groups, each run by a kernel of its own and each longest first: problems with
+    // symmetry orbits, without and with the Lambert column, then the others (and all in mixed precision)
+    // alike.  A fit takes the form that ps_fit_batch gives it, whatever else is in the batch.
+    auto group = [&](int j) {
+        const ps_handle *h = b->hs[prob[j]];
+        return (b->mixed || !h->orbit ? 2 : 0) + int(h->ls);
+    };
     std::vector<int> order(njobs);
     for (int j = 0; j < njobs; ++j) order[j] = j;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        const bool lx = b->hs[prob[x]]->ls, ly = b->hs[prob[y]]->ls;
-        if (lx != ly) return ly;
+        const int gx = group(x), gy = group(y);
+        if (gx != gy) return gx < gy;
         return b->cost[prob[x]] > b->cost[prob[y]];
     });
     std::vector<psk::QueueJob> jobs(njobs);
-    int n0 = 0;
+    int first[5] = {0, 0, 0, 0, njobs};  // the groups' places in jobs
     for (int k = 0; k < njobs; ++k) {
         const int j = order[k];
         jobs[k] = {freq[j], prob[j], pole[j], j, 0};
-        n0 += !b->hs[prob[j]]->ls;
+        for (int g = group(j) + 1; g < 4; ++g) first[g] = k + 1;
     }
-    const int n1 = njobs - n0;
+    const int norbit = first[2];  // jobs of the orbit form
     if (njobs > b->cap_jobs) {
         if (b->exec) hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
@@ -1492,12 +1495,12 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     // (10 to 100 iterations, mean 33) 10240 fits of 512 asteroids in 44 pieces took 2073 ms spread
     // against 746 ms queued, so then only what fits one piece is spread.
     bool spread = false;
-    if (b->orbit) {
+    if (norbit > 0) {
         double sum = 0, longest = 0;
         long passes = 0;
         bool early = false;
-        for (int j = 0; j < njobs; ++j) {
-            const ps_handle *h = b->hs[prob[j]];
+        for (int k = 0; k < norbit; ++k) {
+            const ps_handle *h = b->hs[jobs[k].prob];
             passes += h->P2.npass;
             early |= h->P.iter_diff_max > 0;
             const double w = double(h->P2.npass) * h->nfac / 288;
@@ -1518,57 +1521,55 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
         for (int part = 0; part < 2 && spread; ++part) {
             std::vector<psk::SpreadJob> sj;
             std::vector<int> iters;
-            for (int k = part ? n0 : 0; k < (part ? njobs : n0); ++k) {
+            for (int k = first[part]; k < first[part + 1]; ++k) {
                 const ps_handle *h = b->hs[jobs[k].prob];
                 sj.push_back(spread_job(h, jobs[k].freq, jobs[k].pole, conw_r[jobs[k].prob], jobs[k].out));
                 iters.push_back(iteration_cap(h));
             }
             if (sj.empty()) continue;
-            if (part && n0) HIPCHECK(hipStreamSynchronize(b->stream));  // the first part's tables
+            if (part && first[1]) HIPCHECK(hipStreamSynchronize(b->stream));  // the first part's tables
             rc = spread_fits(b->spread, b->stream, sj, iters, part == 1, b->slots, mfit, nfac, b->d_out);
             if (rc < 0) return rc;
             if (rc == 1) spread = false;  // no memory for it: the queue runs everything
         }
-        if (spread) HIPCHECK(hipEventRecord(b->ev1, b->stream));
     }
-    if (!spread) {
+    const int queued = spread ? norbit : 0;  // the first job of the queue
+    if (queued < njobs) {
         HIPCHECK(hipMemcpyAsync(b->d_conw, conw_r, sizeof(double) * nh, hipMemcpyHostToDevice, b->stream));
         HIPCHECK(hipMemcpyAsync(b->d_jobs, jobs.data(), sizeof(psk::QueueJob) * njobs, hipMemcpyHostToDevice, b->stream));
-        if (!b->exec || b->exec_n0 != n0 || b->exec_n1 != n1) {
+        std::array<int, 5> key{queued};
+        for (int g = 0; g < 4; ++g) key[1 + g] = std::max(0, first[g + 1] - std::max(first[g], queued));
+        if (!b->exec || b->exec_key != key) {
             if (b->exec) hipGraphExecDestroy(b->exec);
             b->exec = nullptr;
             hipGraph_t g = nullptr;
             HIPCHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            hipLaunchKernelGGL(psk::queue_reset, dim3(1), dim3(64), 0, b->stream, b->d_counter, 2);
-            if (b->mixed) {
-                if (n0)
-                    hipLaunchKernelGGL(psk::queue_kernel_mixed<false>, dim3(std::min(n0, b->slots)), dim3(kWG), 0, b->stream,
-                                       b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs, n0, b->d_counter, b->d_out);
-                if (n1)
-                    hipLaunchKernelGGL(psk::queue_kernel_mixed<true>, dim3(std::min(n1, b->slots)), dim3(kWG), 0, b->stream,
-                                       b->d_probs, b->d_layout, b->d_conw, b->lpool, b->d_jobs + n0, n1, b->d_counter + 1,
+            hipLaunchKernelGGL(psk::queue_reset, dim3(1), dim3(64), 0, b->stream, b->d_counter, 4);
+            auto launch = [&](auto *kern, const auto &pool, int wg, int gr) {
+                if (key[1 + gr])
+                    hipLaunchKernelGGL(kern, dim3(std::min(key[1 + gr], b->slots)), dim3(wg), 0, b->stream, b->d_probs,
+                                       b->d_layout, b->d_conw, pool, b->d_jobs + first[gr], key[1 + gr], b->d_counter + gr,
                                        b->d_out);
+            };
+            if (b->mixed) {
+                launch(psk::queue_kernel_mixed<false>, b->lpool, kWG, 2);
+                launch(psk::queue_kernel_mixed<true>, b->lpool, kWG, 3);
             } else {
-                auto launch = [&](auto *kern, int njob, const psk::QueueJob *job, int *counter) {
-                    if (njob)
-                        hipLaunchKernelGGL(kern, dim3(std::min(njob, b->slots)), dim3(psk::kWG2), 0, b->stream, b->d_probs,
-                                           b->d_layout, b->d_conw, b->pool, job, njob, counter, b->d_out);
-                };
-                launch(b->orbit ? psk::queue_kernel2<true, false> : psk::queue_kernel2<false, false>, n0, b->d_jobs, b->d_counter);
-                launch(b->orbit ? psk::queue_kernel2<true, true> : psk::queue_kernel2<false, true>, n1, b->d_jobs + n0,
-                       b->d_counter + 1);
+                launch(psk::queue_kernel2<true, false>, b->pool, psk::kWG2, 0);
+                launch(psk::queue_kernel2<true, true>, b->pool, psk::kWG2, 1);
+                launch(psk::queue_kernel2<false, false>, b->pool, psk::kWG2, 2);
+                launch(psk::queue_kernel2<false, true>, b->pool, psk::kWG2, 3);
             }
             hipError_t e = hipStreamEndCapture(b->stream, &g);
             if (e == hipSuccess) e = hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0);
             if (g) hipGraphDestroy(g);
             if (e != hipSuccess) return ps_fail(PS_ERR_DEVICE, "ps_batch_run: graph capture failed: %s", hipGetErrorString(e));
-            b->exec_n0 = n0;
-            b->exec_n1 = n1;
+            b->exec_key = key;
         }
-        HIPCHECK(hipEventRecord(b->ev0, b->stream));
+        if (!spread) HIPCHECK(hipEventRecord(b->ev0, b->stream));
         HIPCHECK(hipGraphLaunch(b->exec, b->stream));
-        HIPCHECK(hipEventRecord(b->ev1, b->stream));
     }
+    HIPCHECK(hipEventRecord(b->ev1, b->stream));
     HIPCHECK(hipMemcpyAsync(out, b->d_out, sizeof(ps_fit_result) * njobs, hipMemcpyDeviceToHost, b->stream));
     HIPCHECK(hipStreamSynchronize(b->stream));
     float ms = 0;

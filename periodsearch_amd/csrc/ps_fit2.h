@@ -1318,7 +1318,7 @@ struct QueueJob {
     int pad;
 };
 
-// ORBIT: every problem of the batch has symmetry orbits (the layout is then its OrbitModel's, Lmax 3-6).
+// ORBIT: the problems of the jobs have symmetry orbits (the layout is then the OrbitModel's, Lmax 3-6).
 template <bool ORBIT, bool LS>
 __global__ __launch_bounds__(kWG2, 2) void queue_kernel2(const DevProblem *const *probs, const int *layout,
                                                          const double *conw, Slots2 S, const QueueJob *jobs, int njobs,
