@@ -101,8 +101,9 @@ __device__ inline void curv2(const DevProblem &P, const double *a, Shared2<NFM> 
 
 // The same into the orbit form's table: facet i's entry, negated for the member -n_k of its pair.  With
 // LS the second number is Area (the loop multiplies it by cls and sums the Lambert columns from it).  The
-// table is scaled by a power of two so that its largest number is about 1 (a runaway Lambert weight or
-// shape would leave the range of the correction's FP32); the row sums are scaled back by sh.ascale.
+// table is scaled by a power of two so that its largest number, Area*cls included, is about 1 (a runaway
+// weight of the scattering law or shape would leave the range of the correction's FP32); the row sums are
+// scaled back by sh.ascale.
 template <bool LS, int NFM>
 __device__ inline void curv_orbit(const DevProblem &P, const double *a, Shared2<NFM> &sh, double *area) {
     constexpr int kPer = (NFM + kWG2 - 1) / kWG2;  // facets per lane
@@ -117,6 +118,7 @@ __device__ inline void curv_orbit(const DevProblem &P, const double *a, Shared2<
             if (area) area[i] = ar;
             t0[k] = ar * cl;
             t1[k] = LS ? ar : ar * cls;
+            if constexpr (LS) big = fmax(big, fabs(ar * cls));
         }
         big = fmax(big, fmax(fabs(t0[k]), fabs(t1[k])));
     }

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from periodsearch_amd import PS_KERNEL_JFREE, PeriodSearch
+from tests import oracle_binding as ob
 from tests.test_gpu_orbits import problem
 
 pytestmark = pytest.mark.gpu
@@ -49,5 +50,36 @@ def test_raw_rows_of_part_filled_passes(shape):
             got = ps.eval(vecs[:m], conw, raw=True)
             for k in KEYS:
                 assert np.array_equal(got[k], full[k][:m]), (m, k)
+    finally:
+        ps.close()
+
+
+@pytest.mark.parametrize("cl_free", [False, True])
+@pytest.mark.parametrize("cls", [1e45, 1e100, 1e-45])
+def test_any_lommel_seeliger_weight(cls, cl_free):
+    """The caller's vector may hold any weight of the Lommel-Seeliger term: with raw rows (whose Lambert columns
+    keep the weight apart from the areas) as without."""
+    text = problem(6, 6, 6, 2, 50, 300, cl_free=cl_free)
+    orc = ob.OracleCtx.from_text(text)
+    ps = prepared(6, 6, 6, 2, 50, 300, cl_free=cl_free)
+    try:
+        conw = ps.info()["conw_r0"]
+        orc.set_conw(conw)
+        vecs = vectors(ps, 3)
+        vecs[:, -1] = cls
+        got, plain = ps.eval(vecs, conw, raw=True), ps.eval(vecs, conw)
+        for k in ("alpha", "beta", "chisq"):
+            assert np.array_equal(got[k], plain[k]), k
+        arr = ps.input_arrays()
+        n = len(arr["tim"])
+        for v, a in enumerate(vecs):
+            al, be, chi = orc.mrqcof(a)
+            assert np.abs(got["alpha"][v] - al).max() <= 1e-11 * np.abs(al).max()
+            assert np.abs(got["beta"][v] - be).max() <= 1e-11 * np.abs(be).max()
+            assert abs(got["chisq"][v] - chi) <= 1e-12 * chi
+            for p in (0, n // 3, n - 1):
+                br, dy = orc.bright(a, arr["ee"][p], arr["ee0"][p], arr["tim"][p])
+                assert abs(got["ymod"][v, p] - br) <= 1e-13 * abs(br), p
+                assert np.abs(got["dyda"][v, p] - dy).max() <= 1e-12 * np.abs(dy).max(), p
     finally:
         ps.close()
