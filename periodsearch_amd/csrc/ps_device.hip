@@ -1206,12 +1206,13 @@ extern "C" int ps_set_kernel(ps_handle *h, int kernel) {
 }
 
 namespace {
-// Kernel forms chosen by ps_autotune, per problem shape, for the life of the process.
+// Kernel forms chosen by ps_autotune, per problem shape, for the life of the process.  The shape includes
+// what the J-free form's cost depends on beside the sizes: whether the mesh has symmetry orbits (about
+// twice the speed) and the number of passes the lightcurves pack into.
 struct TuneKey {
-    int ncoef, nfac, npts, mfit, ls, iters;
-    bool operator<(const TuneKey &o) const {
-        return std::tie(ncoef, nfac, npts, mfit, ls, iters) < std::tie(o.ncoef, o.nfac, o.npts, o.mfit, o.ls, o.iters);
-    }
+    int ncoef, nfac, npts, mfit, ls, iters, orbit, npass;
+    auto tie() const { return std::tie(ncoef, nfac, npts, mfit, ls, iters, orbit, npass); }
+    bool operator<(const TuneKey &o) const { return tie() < o.tie(); }
 };
 std::map<TuneKey, std::array<double, 2>> g_tuned;  // ms per fit of the two forms
 std::mutex g_tuned_mu;
@@ -1222,7 +1223,7 @@ extern "C" int ps_autotune(ps_handle *h, double conw_r, int *kernel, double *ms_
     std::array<double, 2> ms{0, 0};
     int choice = PS_KERNEL_LEGACY;
     if (h->precision == PS_FP64 && h->v2) {
-        const TuneKey key{h->ncoef, h->nfac, h->npts, h->mfit, int(h->ls), h->P.n_iter_max};
+        const TuneKey key{h->ncoef, h->nfac, h->npts, h->mfit, int(h->ls), h->P.n_iter_max, h->orbit, h->P2.npass};
         bool known = false;
         {
             std::lock_guard<std::mutex> lk(g_tuned_mu);
