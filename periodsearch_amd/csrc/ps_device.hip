@@ -342,6 +342,7 @@ struct ps_handle {
         std::vector<hipEvent_t> chunk, slot;
     } ev;
     Spread spread;
+    int last_spread = 0;  // fits or vectors of the last call that took the spread form
     std::vector<double> wq2_host;
     double *d_wq2 = nullptr;
     std::vector<void *> owned;
@@ -856,11 +857,22 @@ double spread_time(const std::vector<psk::SpreadJob> &jobs, int q, int slots) {
     return tasks <= slots / 2 ? per : kSpreadPaired * double((tasks + slots - 1) / slots) * per;
 }
 
-std::vector<psk::SpreadTask> spread_tasks(const std::vector<psk::SpreadJob> &jobs, int slots) {
+int spread_length(const std::vector<psk::SpreadJob> &jobs, int slots) {  // the passes to a task that take least time
     int longest = 1, best = 1;
     for (const auto &j : jobs) longest = std::max(longest, j.npass);
-    for (int q = 2; q <= longest; ++q)
-        if (spread_time(jobs, q, slots) < spread_time(jobs, best, slots)) best = q;
+    double least = spread_time(jobs, 1, slots);
+    for (int q = 2; q <= longest; ++q) {
+        const double t = spread_time(jobs, q, slots);
+        if (t < least) {
+            least = t;
+            best = q;
+        }
+    }
+    return best;
+}
+
+std::vector<psk::SpreadTask> spread_tasks(const std::vector<psk::SpreadJob> &jobs, int slots) {
+    const int best = spread_length(jobs, slots);
     std::vector<psk::SpreadTask> tasks;
     for (int j = 0; j < int(jobs.size()); ++j) {
         const int np = jobs[j].npass, n = (np + best - 1) / best;  // tasks of equal length, give or take a pass
@@ -964,10 +976,45 @@ psk::SpreadJob spread_job(const ps_handle *h, double freq, int pole, double conw
 }
 int iteration_cap(const ps_handle *h) { return std::max({h->P.n_iter_max, h->P.n_iter_min, 0}); }
 
-// Up to this share of the resident workgroups, fits are spread: one workgroup each would leave so much of
-// the chip idle that two launches per iteration and the solves' latency cost less (figures: ps_spread.h).
+// Whether n fits (or, evals, single evaluations) of a problem are faster spread than in one workgroup each,
+// in us an iteration.  Both forms pay for the solve; a workgroup of its own walks all passes, two to a CU
+// 1.5 times as long; the spread form takes spread_time and its launches and trips through memory: 14 us
+// and what the solves' workgroups read, or, for evaluations, 33 us (the jobs' and tasks' upload included)
+// and the tables' making.  The time of a pass, a fit over 3 + 0.1 mfit + norb (0.2 + 0.003 N): measured 8.9
+// (Lmax 2, 128 facets), 14.5 (3, 288), 13 (4, 200), 21 (6, 288), 30.5 (6, 512).
+// Measured on both sides of the rule, one workgroup each / spread, us for 6 iterations: Lmax 6, 288 facets,
+// 10 fits of 1 pass 484 / 590, 2 passes 632 / 586; 200 fits of 4 passes 934 / 994, 10 passes 1816 / 1637;
+// 281 fits of 4 passes 1203 / 1540, 10 passes 2496 / 2212; Lmax 2, 128 facets, 10 fits of 2 passes 263 / 294,
+// 3 passes 325 / 284; one evaluation at Lmax 3, 288 facets, of 2 passes 75 / 97, 6 passes 132 / 91.
+// From 0.55 of the resident workgroups on, the tasks take too many rounds (figures: ps_spread.h).
 constexpr double kSpreadShare = 0.55;
+bool spread_pays(const ps_handle *h, int n, bool evals) {
+    const int np = h->P2.npass;
+    if (!h->orbit || np < 2 || n > kSpreadShare * h->slots2) return false;
+    const double pass = 3 + 0.1 * h->mfit + h->P2.norb * (0.2 + 0.003 * psk::orb_ncoef(h->orbit));
+    const double solo = pass * (np + kSpreadSetup) * (n > h->slots2 / 2 ? kSpreadPaired : 1.0);
+    double spread = 0;
+    for (int left = n, most = std::max(1, kSpreadPasses / np); left > 0; left -= most) {  // piece by piece
+        const std::vector<psk::SpreadJob> jobs(std::min(left, most), spread_job(h, 0, 0, 0, 0));
+        const int q = spread_length(jobs, h->slots2);
+        spread += pass * spread_time(jobs, q, h->slots2);
+        spread += evals ? 33 + 0.012 * jobs.size() * ((np + q - 1) / q) : 14 + 1.7e-5 * jobs.size() * h->mfit * h->mfit;
+    }
+    return (evals ? 1.1 : 1.05) * spread < solo;
+}
+
+// The fits of a list that are spread: those past whole rounds of the resident workgroups.  A piece of spread
+// fits lasts as long as its slowest fit, and a workgroup of its own that is done goes on to the next fit of
+// the list: where fits may stop early, only a list that is short of a round and fits one piece is spread
+// (712 fits of 10 - 15 iterations, 10 passes, Lmax 6: 7.3 ms in rounds, 8.0 ms with the last 200 spread).
+int spread_rest(const ps_handle *h, int nfits) {
+    const int rest = nfits % h->slots2;
+    if (h->P.iter_diff_max > 0 && (rest < nfits || long(rest) * h->P2.npass > kSpreadPasses)) return 0;
+    return spread_pays(h, rest, false) ? rest : 0;
+}
 }  // namespace
+
+extern "C" int ps_test_spread(const ps_handle *h) { return h->last_spread; }
 
 extern "C" int ps_set_precision(ps_handle *h, int precision) {
     if (!h) return ps_fail(PS_ERR_ARG, "ps_set_precision: null handle");
@@ -1018,30 +1065,31 @@ int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, d
     int rc = set_conw(h, conw_r);
     if (rc != PS_OK) return rc;
     // the last fits, short of a round
-    int rest = 0;
-    if (spread && use_v2(h) && h->orbit) {
-        rest = nfits % h->slots2;
-        if (rest > kSpreadShare * h->slots2) rest = 0;
-    }
+    int rest = spread && use_v2(h) ? spread_rest(h, nfits) : 0;
     int main = nfits - rest;
     if (main > 0) {
         rc = ensure_scratch(h, use_v2(h));
         if (rc != PS_OK) return rc;
     }
-    HIPCHECK(hipMemcpyAsync(h->d_freq, freq, sizeof(double) * nfits, hipMemcpyHostToDevice, h->stream));
-    HIPCHECK(hipMemcpyAsync(h->d_pole, pole, sizeof(int) * nfits, hipMemcpyHostToDevice, h->stream));
-    HIPCHECK(hipEventRecord(h->ev0, h->stream));
     if (rest > 0) {
+        HIPCHECK(hipEventRecord(h->ev0, h->stream));
         std::vector<psk::SpreadJob> jobs(rest);
         for (int i = 0; i < rest; ++i) jobs[i] = spread_job(h, freq[main + i], pole[main + i], conw_r, main + i);
         rc = spread_fits(h->spread, h->stream, jobs, std::vector<int>(rest, iteration_cap(h)), h->ls, h->slots2, h->mfit,
                          h->nfac, h->d_out);
         if (rc < 0) return rc;
         if (rc == 1) {
+            rest = 0;
             main = nfits;
             rc = ensure_scratch(h, true);
             if (rc != PS_OK) return rc;
         }
+    }
+    h->last_spread = rest;
+    if (main > 0) {
+        HIPCHECK(hipMemcpyAsync(h->d_freq, freq, sizeof(double) * nfits, hipMemcpyHostToDevice, h->stream));
+        HIPCHECK(hipMemcpyAsync(h->d_pole, pole, sizeof(int) * nfits, hipMemcpyHostToDevice, h->stream));
+        if (rest == 0) HIPCHECK(hipEventRecord(h->ev0, h->stream));
     }
     if (main == 0) {
     } else if (use_v2(h)) {
@@ -1621,8 +1669,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     int rc = set_conw(h, conw_r);
     if (rc != PS_OK) return rc;
     // few vectors: their passes spread over the chip
-    bool spread = use_v2(h) && h->orbit && h->P2.npass > 1 && nvec <= kSpreadShare * h->slots2 &&
-                  long(nvec) * h->P2.npass <= kSpreadPasses;
+    bool spread = use_v2(h) && long(nvec) * h->P2.npass <= kSpreadPasses && spread_pays(h, nvec, true);
     std::vector<psk::SpreadJob> sjobs;
     std::vector<psk::SpreadTask> stasks;
     if (spread) {
@@ -1633,6 +1680,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         stasks = spread_tasks(sjobs, h->slots2);
         spread = spread_buffers(h->spread, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac);
     }
+    h->last_spread = spread ? nvec : 0;
     if (!spread) {
         rc = ensure_scratch(h, use_v2(h));
         if (rc != PS_OK) return rc;
