@@ -1007,8 +1007,10 @@ bool spread_pays(const ps_handle *h, int n, bool evals) {
 // fits lasts as long as its slowest fit, and a workgroup of its own that is done goes on to the next fit of
 // the list: where fits may stop early, only a list that is short of a round and fits one piece is spread
 // (712 fits of 10 - 15 iterations, 10 passes, Lmax 6: 7.3 ms in rounds, 8.0 ms with the last 200 spread).
+// Fits of no iteration (stop 1, minimum 0) evaluate nothing; the spread form would evaluate the start.
 int spread_rest(const ps_handle *h, int nfits) {
     const int rest = nfits % h->slots2;
+    if (iteration_cap(h) < 1) return 0;
     if (h->P.iter_diff_max > 0 && (rest < nfits || long(rest) * h->P2.npass > kSpreadPasses)) return 0;
     return spread_pays(h, rest, false) ? rest : 0;
 }
@@ -1547,18 +1549,19 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     if (norbit > 0) {
         double sum = 0, longest = 0;
         long passes = 0;
-        bool early = false;
+        bool early = false, idle = false;
         for (int k = 0; k < norbit; ++k) {
             const ps_handle *h = b->hs[jobs[k].prob];
             passes += h->P2.npass;
             early |= h->P.iter_diff_max > 0;
+            idle |= iteration_cap(h) < 1;  // a fit of no iteration: spread_rest
             const double w = double(h->P2.npass) * h->nfac / 288;
             sum += w;
             longest = std::max(longest, w);
         }
         const double share = kSpreadPaired * sum / b->slots;
         const long pieces = (passes + kSpreadPasses - 1) / kSpreadPasses;
-        spread = share * 1.1 + 3 * pieces < std::max(longest, share + 0.5 * longest) && (!early || pieces == 1);
+        spread = share * 1.1 + 3 * pieces < std::max(longest, share + 0.5 * longest) && (!early || pieces == 1) && !idle;
     }
     if (spread) {
         size_t mfit = 1, nfac = 1;

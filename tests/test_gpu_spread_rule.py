@@ -7,7 +7,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from periodsearch_amd import FIT_DTYPE, PS_KERNEL_JFREE, PeriodSearch, lib, synth
+from periodsearch_amd import FIT_DTYPE, PS_KERNEL_JFREE, Batch, PeriodSearch, lib, synth
 from tests.test_gpu_orbits import problem
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +94,19 @@ def test_the_shapes_compared_bit_for_bit_are_spread():
                     assert np.array_equal(got[k], full[k][:m], equal_nan=True), (m, k)
         finally:
             ps.close()
+
+
+def test_fits_of_no_iteration_evaluate_nothing():
+    """Stop 1 with a minimum of 0: the driver's loop (period_search_BOINC.cpp:868-872) does not run."""
+    text, _ = synth.generate(synth.config1(stop_condition=1, n_iter_min=0))
+    ps = prepared(text)
+    try:
+        conw = ps.info()["conw_r0"]
+        freq, pole = ps.freq(np.full(10, 2)), np.arange(1, 11)
+        with Batch([ps]) as b:
+            lists = ps.fit_batch(freq, pole, conw), b.run([conw], np.zeros(10), freq, pole)
+        for got in lists:
+            for k in ("niter", "nsolve_fail", "chisq", "dev", "dark"):
+                assert (got[k] == 0).all(), (k, got[k])
+    finally:
+        ps.close()
