@@ -14,11 +14,13 @@
 #include <map>
 #include <tuple>
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/periodsearch_amd.h"
@@ -299,14 +301,19 @@ namespace {
 // Device buffers of the spread form (ps_spread.h), one allocation kept by a handle or batch and grown on
 // demand.  The passes in flight are bounded: longer job lists run in pieces.
 constexpr int kSpreadPasses = 8192;  // 192 MiB of Gram blocks
+struct SpreadPiece {
+    std::vector<psk::SpreadJob> jobs;  // host copies, alive until their uploads have run
+    std::vector<psk::SpreadTask> tasks;
+    int passes = 0, most = 0;  // the most iterations of a job
+};
 struct Spread {
     psk::SpreadBuf B{};
     psk::SpreadJob *jobs = nullptr;
     psk::SpreadTask *tasks = nullptr;
-    std::vector<psk::SpreadJob> hjobs;  // host copies, alive until their uploads have run
-    std::vector<psk::SpreadTask> htasks;
+    std::vector<SpreadPiece> pieces;
     char *arena = nullptr;
     size_t cap = 0;
+    size_t limit = size_t(-1);  // the largest arena that may be had (ps_test_limits)
 };
 }  // namespace
 
@@ -884,89 +891,86 @@ std::vector<psk::SpreadTask> spread_tasks(const std::vector<psk::SpreadJob> &job
     return tasks;
 }
 
-// Buffers for a piece of jobs; false when memory runs out.
-bool spread_buffers(Spread &S, size_t njobs, size_t ntasks, size_t passes, size_t mfit, size_t nfac) {
+// Places the buffers of a piece in the arena (there may be none yet); returns the bytes they take.
+size_t spread_layout(Spread &S, size_t njobs, size_t ntasks, size_t passes, size_t mfit, size_t nfac) {
     size_t need = 0;
-    auto place = [&](size_t bytes) {
-        const size_t at = need;
-        need += (bytes + 255) & ~size_t(255);
-        return at;
+    auto place = [&](auto *&p, size_t n) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<uintptr_t>(S.arena) + need);
+        need += (n * sizeof(*p) + 255) & ~size_t(255);
     };
     S.B.a_stride = mfit * mfit;
     S.B.b_stride = mfit;
     S.B.f_stride = nfac;
-    const size_t state = place(njobs * sizeof(psk::SpreadState)), part = place(passes * psk::kStashPerSlot * sizeof(double)),
-                 alpha = place(2 * njobs * S.B.a_stride * sizeof(double)), beta = place(2 * njobs * S.B.b_stride * sizeof(double)),
-                 area = place(2 * njobs * S.B.f_stride * sizeof(double)), done = place(sizeof(int)),
-                 jobs = place(njobs * sizeof(psk::SpreadJob)), tasks = place(ntasks * sizeof(psk::SpreadTask));
-    if (need > S.cap) {
-        (void)hipFree(S.arena);
-        S.cap = 0;
-        if (hipMalloc(&S.arena, need) != hipSuccess) {
-            (void)hipGetLastError();
-            S.arena = nullptr;
-            return false;
-        }
-        S.cap = need;
+    place(S.B.state, njobs);
+    place(S.B.part, passes * psk::kStashPerSlot);
+    place(S.B.alpha, 2 * njobs * S.B.a_stride);
+    place(S.B.beta, 2 * njobs * S.B.b_stride);
+    place(S.B.area, 2 * njobs * S.B.f_stride);
+    place(S.B.done, 1);
+    place(S.jobs, njobs);
+    place(S.tasks, ntasks);
+    return need;
+}
+
+// An arena of the given size; false when it cannot be had.
+bool spread_reserve(Spread &S, size_t need) {
+    if (need <= S.cap) return true;
+    (void)hipFree(S.arena);
+    S.arena = nullptr;
+    S.cap = 0;
+    if (need > S.limit || hipMalloc(&S.arena, need) != hipSuccess) {
+        (void)hipGetLastError();
+        S.arena = nullptr;
+        return false;
     }
-    auto at = [&](size_t o) { return reinterpret_cast<double *>(S.arena + o); };
-    S.B.state = reinterpret_cast<psk::SpreadState *>(S.arena + state);
-    S.B.part = at(part);
-    S.B.alpha = at(alpha);
-    S.B.beta = at(beta);
-    S.B.area = at(area);
-    S.B.done = reinterpret_cast<int *>(S.arena + done);
-    S.jobs = reinterpret_cast<psk::SpreadJob *>(S.arena + jobs);
-    S.tasks = reinterpret_cast<psk::SpreadTask *>(S.arena + tasks);
+    S.cap = need;
     return true;
 }
 
 // Runs the fits of jobs (all with or all without the Lambert column) on the stream; results to d_out.
-// Returns 1 when the buffers cannot be had and nothing has run (the caller then takes the other form).
+// Returns 1 when the buffers cannot be had and nothing has run (the caller then takes the other form):
+// those of all pieces are taken before the first one starts.
 int spread_fits(Spread &S, hipStream_t stream, const std::vector<psk::SpreadJob> &all, const std::vector<int> &iters,
                 bool ls, int slots, size_t mfit, size_t nfac, ps_fit_result *d_out) {
     constexpr int kCheck = 16;  // iterations launched between looks at the number of finished fits
-    for (size_t i0 = 0; i0 < all.size();) {
-        if (i0 > 0) HIPCHECK(hipStreamSynchronize(stream));  // the piece before still reads its tables
-        auto &jobs = S.hjobs;
-        jobs.clear();
-        int passes = 0, most = 0;
-        size_t i = i0;
-        for (; i < all.size() && (i == i0 || passes + all[i].npass <= kSpreadPasses); ++i) {
-            jobs.push_back(all[i]);
-            jobs.back().part0 = passes;
-            passes += all[i].npass;
-            most = std::max(most, iters[i]);
+    S.pieces.clear();
+    size_t need = 0;
+    for (size_t i = 0; i < all.size();) {
+        auto &p = S.pieces.emplace_back();
+        for (const size_t i0 = i; i < all.size() && (i == i0 || p.passes + all[i].npass <= kSpreadPasses); ++i) {
+            p.jobs.push_back(all[i]);
+            p.jobs.back().part0 = p.passes;
+            p.passes += all[i].npass;
+            p.most = std::max(p.most, iters[i]);
         }
-        auto &tasks = S.htasks;
-        tasks = spread_tasks(jobs, slots);
-        if (!spread_buffers(S, jobs.size(), tasks.size(), passes, mfit, nfac)) {
-            if (i0 == 0) return 1;
-            return ps_fail(PS_ERR_NOMEM, "scratch allocation failed (%zu fits)", jobs.size());
-        }
-        HIPCHECK(hipMemcpyAsync(S.jobs, jobs.data(), sizeof(jobs[0]) * jobs.size(), hipMemcpyHostToDevice, stream));
-        HIPCHECK(hipMemcpyAsync(S.tasks, tasks.data(), sizeof(tasks[0]) * tasks.size(), hipMemcpyHostToDevice, stream));
-        const int nj = int(jobs.size());
+        p.tasks = spread_tasks(p.jobs, slots);
+        need = std::max(need, spread_layout(S, p.jobs.size(), p.tasks.size(), p.passes, mfit, nfac));
+    }
+    if (!spread_reserve(S, need)) return 1;
+    for (const auto &p : S.pieces) {  // one after the other on the stream
+        spread_layout(S, p.jobs.size(), p.tasks.size(), p.passes, mfit, nfac);
+        HIPCHECK(hipMemcpyAsync(S.jobs, p.jobs.data(), sizeof(p.jobs[0]) * p.jobs.size(), hipMemcpyHostToDevice, stream));
+        HIPCHECK(hipMemcpyAsync(S.tasks, p.tasks.data(), sizeof(p.tasks[0]) * p.tasks.size(), hipMemcpyHostToDevice, stream));
+        const int nj = int(p.jobs.size());
         hipLaunchKernelGGL(psk::spread_reset, dim3((nj + 255) / 256), dim3(256), 0, stream, S.B, nj);
         hipLaunchKernelGGL(psk::spread_step, dim3(nj), dim3(psk::kWG2), 0, stream, S.jobs, S.B, d_out);
-        for (int it = 0; it <= most;) {  // the starting point and every iteration's trial point
-            for (int c = 0; c < kCheck && it <= most; ++c, ++it) {
+        for (int it = 0; it <= p.most;) {  // the starting point and every iteration's trial point
+            for (int c = 0; c < kCheck && it <= p.most; ++c, ++it) {
                 if (ls)
-                    hipLaunchKernelGGL(psk::spread_eval<true>, dim3(tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs, S.tasks,
-                                       S.B, nullptr, nullptr, nullptr);
+                    hipLaunchKernelGGL(psk::spread_eval<true>, dim3(p.tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs,
+                                       S.tasks, S.B, nullptr, nullptr, nullptr);
                 else
-                    hipLaunchKernelGGL(psk::spread_eval<false>, dim3(tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs, S.tasks,
-                                       S.B, nullptr, nullptr, nullptr);
+                    hipLaunchKernelGGL(psk::spread_eval<false>, dim3(p.tasks.size()), dim3(psk::kWG2), 0, stream, S.jobs,
+                                       S.tasks, S.B, nullptr, nullptr, nullptr);
                 hipLaunchKernelGGL(psk::spread_step, dim3(nj), dim3(psk::kWG2), 0, stream, S.jobs, S.B, d_out);
             }
             if (hipGetLastError() != hipSuccess) return ps_fail(PS_ERR_DEVICE, "spread fit launch failed");
-            if (it > most) break;
+            if (it > p.most) break;
             int done = 0;
             HIPCHECK(hipMemcpyAsync(&done, S.B.done, sizeof(int), hipMemcpyDeviceToHost, stream));
             HIPCHECK(hipStreamSynchronize(stream));
             if (done == nj) break;
         }
-        i0 = i;
     }
     return PS_OK;
 }
@@ -1017,6 +1021,7 @@ int spread_rest(const ps_handle *h, int nfits) {
 }  // namespace
 
 extern "C" int ps_test_spread(const ps_handle *h) { return h->last_spread; }
+extern "C" void ps_test_limits(ps_handle *h, size_t arena) { h->spread.limit = arena; }
 
 extern "C" int ps_set_precision(ps_handle *h, int precision) {
     if (!h) return ps_fail(PS_ERR_ARG, "ps_set_precision: null handle");
@@ -1337,6 +1342,7 @@ extern "C" int ps_get_kernel(const ps_handle *h) {
 struct ps_batch {
     int device = 0;
     Spread spread;
+    int last_spread = 0;  // fits of the last run that took the spread form
     std::vector<ps_handle *> hs;
     std::vector<double> cost;  // estimated work of one fit of each problem
     hipStream_t stream = nullptr;
@@ -1585,7 +1591,7 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
             if (rc == 1) spread = false;  // no memory for it: the queue runs everything
         }
     }
-    const int queued = spread ? norbit : 0;  // the first job of the queue
+    const int queued = b->last_spread = spread ? norbit : 0;  // the first job of the queue
     if (queued < njobs) {
         HIPCHECK(hipMemcpyAsync(b->d_conw, conw_r, sizeof(double) * nh, hipMemcpyHostToDevice, b->stream));
         HIPCHECK(hipMemcpyAsync(b->d_jobs, jobs.data(), sizeof(psk::QueueJob) * njobs, hipMemcpyHostToDevice, b->stream));
@@ -1630,6 +1636,9 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     b->launches += 1;
     return PS_OK;
 }
+
+extern "C" int ps_test_batch_spread(const ps_batch *b) { return b->last_spread; }
+extern "C" void ps_test_batch_limits(ps_batch *b, size_t arena) { b->spread.limit = arena; }
 
 extern "C" int ps_batch_kernel_time(ps_batch *b, double *ms, int *launches, int reset) {
     if (!b) return ps_fail(PS_ERR_ARG, "ps_batch_kernel_time: null batch");
@@ -1681,7 +1690,11 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
             sjobs.back().part0 = v * h->P2.npass;
         }
         stasks = spread_tasks(sjobs, h->slots2);
-        spread = spread_buffers(h->spread, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac);
+        auto layout = [&] {
+            return spread_layout(h->spread, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac);
+        };
+        spread = spread_reserve(h->spread, layout());
+        if (spread) layout();
     }
     h->last_spread = spread ? nvec : 0;
     if (!spread) {

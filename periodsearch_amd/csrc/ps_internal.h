@@ -2,13 +2,20 @@
 // libpsamd.so.  Not part of the public ABI.
 #pragma once
 
+#include <cstddef>
+
 struct ps_handle;
+struct ps_batch;
 
 // Records a message for ps_last_error() and returns code.
 int ps_fail(int code, const char *fmt, ...);
 
-// For the tests, which pin the route that a call took.
+// For the tests, which pin the route that a call took and what it does at the limits of memory.
 extern "C" {
-// The fits (ps_fit_batch, ps_scan) or vectors (ps_eval) of the handle's last call that took the spread form.
+// The fits (ps_fit_batch, ps_scan, ps_batch_run) or vectors (ps_eval) of the last call that took the spread form.
 int ps_test_spread(const ps_handle *h);
+int ps_test_batch_spread(const ps_batch *b);
+// Caps what later calls can have: bytes of device memory for the spread form's buffers.
+void ps_test_limits(ps_handle *h, size_t arena);
+void ps_test_batch_limits(ps_batch *b, size_t arena);
 }

@@ -1,0 +1,83 @@
+"""Calls whose buffers cannot be had (the limits are forced on the handle or batch): they take the other form and
+return the same bits, as they did before there was a choice of forms."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from periodsearch_amd import FIT_DTYPE, Batch, lib
+from tests.test_gpu_spread_rule import passes, prepared, spread
+
+pytestmark = pytest.mark.gpu
+
+
+def limit(ps, *args):
+    fn = lib().ps_test_limits
+    fn.argtypes, fn.restype = [C.c_void_p] + [C.c_size_t] * len(args), None
+    fn(ps._handle(), *args)
+
+
+def batch_limit(b, arena):
+    fn = lib().ps_test_batch_limits
+    fn.argtypes, fn.restype = [C.c_void_p, C.c_size_t], None
+    fn(b._b, arena)
+
+
+def batch_spread(b):
+    fn = lib().ps_test_batch_spread
+    fn.argtypes, fn.restype = [C.c_void_p], C.c_int
+    return fn(b._b)
+
+
+def same(a, b, what):
+    for k in FIT_DTYPE.names:
+        assert np.array_equal(a[k], b[k], equal_nan=True), (what, k)
+
+
+def test_a_later_piece_larger_than_the_first():
+    """Long fits fill the first piece, many short ones the second: their normal equations take more memory."""
+    searches = [prepared(passes(6, 6, 24)), prepared(passes(3, 4, 2))]
+    try:
+        conw = np.array([s.info()["conw_r0"] for s in searches])
+        prob = np.repeat([0, 1], [336, 4000])
+        pole = np.arange(len(prob)) % 10 + 1
+        freq = np.concatenate([searches[0].freq(1 + np.arange(336) // 10), searches[1].freq(1 + np.arange(4000) // 10 % 50)])
+        with Batch(searches) as b:
+            free = b.run(conw, prob, freq, pole)
+            assert batch_spread(b) == len(prob), "the case means two pieces"
+        with Batch(searches) as b:
+            batch_limit(b, 300 << 20)  # the first piece needs 220 MB, the second 380
+            got = b.run(conw, prob, freq, pole)
+            assert batch_spread(b) == 0
+        same(got, free, "limited")
+        few = np.arange(330, 350)
+        for i, s in enumerate(searches):
+            sel = few[prob[few] == i]
+            same(free[sel], s.fit_batch(freq[sel], pole[sel], conw[i]), i)
+    finally:
+        for s in searches:
+            s.close()
+
+
+def test_no_room_to_spread():
+    text = passes(6, 6, 10)
+    a, b = prepared(text), prepared(text)
+    try:
+        conw = a.info()["conw_r0"]
+        freq, pole = a.freq(1 + np.arange(20) // 10), 1 + np.arange(20) % 10
+        limit(b, 1 << 20)
+        want, got = a.fit_batch(freq, pole, conw), b.fit_batch(freq, pole, conw)
+        assert (spread(a), spread(b)) == (20, 0)
+        same(got, want, "fits")
+        vec = np.zeros((9, a.info()["ma"]))
+        nc = a.info()["ncoef"]
+        vec[:, :nc], vec[:, nc] = a.geometry()["cg_first"], np.linspace(0.5, 2.5, 9)
+        vec[:, nc + 2] = 2 * np.pi * 24 * a.freq(1)
+        vec[:, nc + 3:] = 0.5, 0.1, -0.5, -2.0, 1.0
+        want, got = a.eval(vec, conw, raw=True), b.eval(vec, conw, raw=True)
+        assert (spread(a), spread(b)) == (9, 0)
+        for k in want:
+            assert np.array_equal(got[k], want[k]), k
+    finally:
+        a.close()
+        b.close()
