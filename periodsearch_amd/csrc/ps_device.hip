@@ -298,8 +298,84 @@ int noalloc_setup(int device) {
 }  // namespace
 
 namespace {
-// Device buffers of the spread form (ps_spread.h), one allocation kept by a handle or batch and grown on
-// demand.  The passes in flight are bounded: longer job lists run in pieces.
+// The device memory of the spread form (ps_spread.h), one arena for each call that runs.  Arenas belong to
+// the device, not to a handle: a survey may keep hundreds of handles open, and 200 MB each would be tens of
+// GB.  A call takes one and gives it back when its stream is done; at most kIdle wait for the next call, and
+// they are freed with the device's last handle.
+class ArenaPool {
+public:
+    struct Arena {
+        char *p = nullptr;
+        size_t size = 0;
+    };
+    Arena take(int device, size_t need) {  // p = nullptr when it cannot be had
+        std::lock_guard<std::mutex> lk(mu_);
+        auto &idle = dev_[device].idle;
+        idle.reserve(kIdle + 1);  // give() then allocates nothing
+        auto fit = idle.end();  // the smallest that is large enough
+        for (auto a = idle.begin(); a != idle.end(); ++a)
+            if (a->size >= need && (fit == idle.end() || a->size < fit->size)) fit = a;
+        Arena got;
+        if (fit != idle.end()) {
+            got = *fit;
+            idle.erase(fit);
+            return got;
+        }
+        drop(idle, 1);  // a larger one takes its place
+        if (hipMalloc(&got.p, need) != hipSuccess) {
+            drop(idle, idle.size());
+            if (hipMalloc(&got.p, need) != hipSuccess) {
+                (void)hipGetLastError();
+                return {};
+            }
+        }
+        got.size = need;
+        return got;
+    }
+    void give(int device, Arena a) {  // no work uses it any more
+        if (!a.p) return;
+        std::lock_guard<std::mutex> lk(mu_);
+        auto &d = dev_[device];
+        d.idle.push_back(a);
+        if (d.handles == 0) drop(d.idle, d.idle.size());
+        while (d.idle.size() > kIdle) drop(d.idle, 1);
+    }
+    void handles(int device, int change) {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto &d = dev_[device];
+        d.handles += change;
+        if (d.handles == 0) drop(d.idle, d.idle.size());
+    }
+    size_t idle_bytes(int device, int *handles) {
+        std::lock_guard<std::mutex> lk(mu_);
+        size_t n = 0;
+        for (const Arena &a : dev_[device].idle) n += a.size;
+        *handles = dev_[device].handles;
+        return n;
+    }
+
+private:
+    static constexpr size_t kIdle = 2;
+    struct Device {
+        std::vector<Arena> idle;
+        int handles = 0;
+    };
+    static void drop(std::vector<Arena> &idle, size_t n) {  // the n smallest
+        for (; n > 0 && !idle.empty(); --n) {
+            auto a = std::min_element(idle.begin(), idle.end(), [](const Arena &x, const Arena &y) { return x.size < y.size; });
+            (void)hipFree(a->p);
+            idle.erase(a);
+        }
+    }
+    std::mutex mu_;
+    std::map<int, Device> dev_;
+};
+ArenaPool &arenas() {
+    static ArenaPool *p = new ArenaPool;  // never destroyed: the runtime may be gone before it
+    return *p;
+}
+
+// One call's share of it.  The passes in flight are bounded: longer job lists run in pieces.
 constexpr int kSpreadPasses = 8192;  // 192 MiB of Gram blocks
 struct SpreadPiece {
     std::vector<psk::SpreadJob> jobs;  // host copies, alive until their uploads have run
@@ -311,9 +387,28 @@ struct Spread {
     psk::SpreadJob *jobs = nullptr;
     psk::SpreadTask *tasks = nullptr;
     std::vector<SpreadPiece> pieces;
-    char *arena = nullptr;
-    size_t cap = 0;
-    size_t limit = size_t(-1);  // the largest arena that may be had (ps_test_limits)
+    const int device;
+    const hipStream_t stream;
+    const size_t limit;  // the largest arena that may be had (ps_test_limits)
+    ArenaPool::Arena arena;
+    bool busy = false;  // work on the stream may still use the arena
+
+    Spread(int device, hipStream_t stream, size_t limit) : device(device), stream(stream), limit(limit) {}
+    Spread(const Spread &) = delete;
+    Spread &operator=(const Spread &) = delete;
+    ~Spread() { reset(); }
+    void reset() {
+        if (arena.p && busy) (void)hipStreamSynchronize(stream);
+        arenas().give(device, arena);
+        arena = {};
+        busy = false;
+    }
+    bool reserve(size_t need) {  // false when it cannot be had
+        if (need <= arena.size) return true;
+        reset();
+        if (need <= limit) arena = arenas().take(device, need);
+        return arena.p != nullptr;
+    }
 };
 }  // namespace
 
@@ -348,7 +443,7 @@ struct ps_handle {
         hipStream_t copy = nullptr;  // outputs of a chunk leave while the next one is computed
         std::vector<hipEvent_t> chunk, slot;
     } ev;
-    Spread spread;
+    size_t spread_limit = size_t(-1);  // of the spread form's memory (ps_test_limits)
     int last_spread = 0;  // fits or vectors of the last call that took the spread form
     std::vector<double> wq2_host;
     double *d_wq2 = nullptr;
@@ -523,6 +618,7 @@ extern "C" int ps_prepare(const ps_input *in, const ps_geometry *geo, int device
 
     auto *h = new ps_handle();
     h->device = device;
+    arenas().handles(device, 1);  // until ps_release
     h->ndata = in->ndata;
     h->npts = in->ndata + 3;
     h->nlc = in->lcurves + 1;
@@ -895,7 +991,7 @@ std::vector<psk::SpreadTask> spread_tasks(const std::vector<psk::SpreadJob> &job
 size_t spread_layout(Spread &S, size_t njobs, size_t ntasks, size_t passes, size_t mfit, size_t nfac) {
     size_t need = 0;
     auto place = [&](auto *&p, size_t n) {
-        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<uintptr_t>(S.arena) + need);
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<uintptr_t>(S.arena.p) + need);
         need += (n * sizeof(*p) + 255) & ~size_t(255);
     };
     S.B.a_stride = mfit * mfit;
@@ -912,26 +1008,11 @@ size_t spread_layout(Spread &S, size_t njobs, size_t ntasks, size_t passes, size
     return need;
 }
 
-// An arena of the given size; false when it cannot be had.
-bool spread_reserve(Spread &S, size_t need) {
-    if (need <= S.cap) return true;
-    (void)hipFree(S.arena);
-    S.arena = nullptr;
-    S.cap = 0;
-    if (need > S.limit || hipMalloc(&S.arena, need) != hipSuccess) {
-        (void)hipGetLastError();
-        S.arena = nullptr;
-        return false;
-    }
-    S.cap = need;
-    return true;
-}
-
-// Runs the fits of jobs (all with or all without the Lambert column) on the stream; results to d_out.
+// Runs the fits of jobs (all with or all without the Lambert column) on S's stream; results to d_out.
 // Returns 1 when the buffers cannot be had and nothing has run (the caller then takes the other form):
 // those of all pieces are taken before the first one starts.
-int spread_fits(Spread &S, hipStream_t stream, const std::vector<psk::SpreadJob> &all, const std::vector<int> &iters,
-                bool ls, int slots, size_t mfit, size_t nfac, ps_fit_result *d_out) {
+int spread_fits(Spread &S, const std::vector<psk::SpreadJob> &all, const std::vector<int> &iters, bool ls, int slots,
+                size_t mfit, size_t nfac, ps_fit_result *d_out) {
     constexpr int kCheck = 16;  // iterations launched between looks at the number of finished fits
     S.pieces.clear();
     size_t need = 0;
@@ -946,7 +1027,9 @@ int spread_fits(Spread &S, hipStream_t stream, const std::vector<psk::SpreadJob>
         p.tasks = spread_tasks(p.jobs, slots);
         need = std::max(need, spread_layout(S, p.jobs.size(), p.tasks.size(), p.passes, mfit, nfac));
     }
-    if (!spread_reserve(S, need)) return 1;
+    if (!S.reserve(need)) return 1;
+    const hipStream_t stream = S.stream;
+    S.busy = true;
     for (const auto &p : S.pieces) {  // one after the other on the stream
         spread_layout(S, p.jobs.size(), p.tasks.size(), p.passes, mfit, nfac);
         HIPCHECK(hipMemcpyAsync(S.jobs, p.jobs.data(), sizeof(p.jobs[0]) * p.jobs.size(), hipMemcpyHostToDevice, stream));
@@ -1021,7 +1104,8 @@ int spread_rest(const ps_handle *h, int nfits) {
 }  // namespace
 
 extern "C" int ps_test_spread(const ps_handle *h) { return h->last_spread; }
-extern "C" void ps_test_limits(ps_handle *h, size_t arena) { h->spread.limit = arena; }
+extern "C" size_t ps_test_arenas(int device, int *handles) { return arenas().idle_bytes(device, handles); }
+extern "C" void ps_test_limits(ps_handle *h, size_t arena) { h->spread_limit = arena; }
 
 extern "C" int ps_set_precision(ps_handle *h, int precision) {
     if (!h) return ps_fail(PS_ERR_ARG, "ps_set_precision: null handle");
@@ -1054,8 +1138,9 @@ extern "C" int ps_get_info(const ps_handle *h, ps_info *info) {
 namespace {
 // Uploads one batch of fits of a problem and launches the fit kernel on the problem's stream, without
 // waiting: the results land in h->d_out.  Validation is the caller's.
-// spread: the fits beyond whole rounds of the resident workgroups may take the spread form.
-int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, double conw_r, bool spread) {
+// spread (may be null): the fits beyond whole rounds of the resident workgroups may take the spread form; it
+// outlives the work on the stream.
+int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, double conw_r, Spread *spread) {
     if (nfits > h->cap_fits) {
         (void)hipFree(h->d_freq);
         (void)hipFree(h->d_pole);
@@ -1082,8 +1167,8 @@ int enqueue_fits(ps_handle *h, int nfits, const double *freq, const int *pole, d
         HIPCHECK(hipEventRecord(h->ev0, h->stream));
         std::vector<psk::SpreadJob> jobs(rest);
         for (int i = 0; i < rest; ++i) jobs[i] = spread_job(h, freq[main + i], pole[main + i], conw_r, main + i);
-        rc = spread_fits(h->spread, h->stream, jobs, std::vector<int>(rest, iteration_cap(h)), h->ls, h->slots2, h->mfit,
-                         h->nfac, h->d_out);
+        rc = spread_fits(*spread, jobs, std::vector<int>(rest, iteration_cap(h)), h->ls, h->slots2, h->mfit, h->nfac,
+                         h->d_out);
         if (rc < 0) return rc;
         if (rc == 1) {
             rest = 0;
@@ -1143,8 +1228,11 @@ extern "C" int ps_fit_batch(ps_handle *h, int nfits, const double *freq, const i
     if (rc != PS_OK) return rc;
     if (!(conw_r > 0)) return ps_fail(PS_ERR_ARG, "ps_fit_batch: conw_r must be positive");
     HIPCHECK(hipSetDevice(h->device));
-    rc = enqueue_fits(h, nfits, freq, pole, conw_r, true);
-    return rc != PS_OK ? rc : collect_fits(h, nfits, out);
+    Spread spread(h->device, h->stream, h->spread_limit);
+    rc = enqueue_fits(h, nfits, freq, pole, conw_r, &spread);
+    if (rc == PS_OK) rc = collect_fits(h, nfits, out);
+    if (rc == PS_OK) spread.busy = false;
+    return rc;
 }
 
 extern "C" int ps_fit_multi(ps_handle *const *hs, int nh, const double *conw_r, int njobs, const int *prob,
@@ -1191,7 +1279,7 @@ extern "C" int ps_fit_multi(ps_handle *const *hs, int nh, const double *conw_r, 
             f[i].push_back(freq[j]);
             pl[i].push_back(pole[j]);
         }
-        rc = enqueue_fits(hs[i], int(jobs[i].size()), f[i].data(), pl[i].data(), conw_r[i], false);
+        rc = enqueue_fits(hs[i], int(jobs[i].size()), f[i].data(), pl[i].data(), conw_r[i], nullptr);
         if (rc != PS_OK) return rc;
     }
     std::vector<ps_fit_result> res;
@@ -1341,7 +1429,7 @@ extern "C" int ps_get_kernel(const ps_handle *h) {
 // ---------------------------------------------------------------------------------------------
 struct ps_batch {
     int device = 0;
-    Spread spread;
+    size_t spread_limit = size_t(-1);
     int last_spread = 0;  // fits of the last run that took the spread form
     std::vector<ps_handle *> hs;
     std::vector<double> cost;  // estimated work of one fit of each problem
@@ -1371,7 +1459,6 @@ extern "C" void ps_batch_release(ps_batch *b) {
     if (b->stream) hipStreamSynchronize(b->stream);
     if (b->exec) hipGraphExecDestroy(b->exec);
     for (void *p : b->owned) hipFree(p);
-    hipFree(b->spread.arena);
     hipFree(b->d_jobs);
     hipFree(b->d_out);
     if (b->ev0) hipEventDestroy(b->ev0);
@@ -1551,6 +1638,7 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     // its slowest fit, while a workgroup of the queue goes on to the next job: where fits may stop early
     // (10 to 100 iterations, mean 33) 10240 fits of 512 asteroids in 44 pieces took 2073 ms spread
     // against 746 ms queued, so then only what fits one piece is spread.
+    Spread S(b->device, b->stream, b->spread_limit);
     bool spread = false;
     if (norbit > 0) {
         double sum = 0, longest = 0;
@@ -1586,7 +1674,7 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
             }
             if (sj.empty()) continue;
             if (part && first[1]) HIPCHECK(hipStreamSynchronize(b->stream));  // the first part's tables
-            rc = spread_fits(b->spread, b->stream, sj, iters, part == 1, b->slots, mfit, nfac, b->d_out);
+            rc = spread_fits(S, sj, iters, part == 1, b->slots, mfit, nfac, b->d_out);
             if (rc < 0) return rc;
             if (rc == 1) spread = false;  // no memory for it: the queue runs everything
         }
@@ -1630,6 +1718,7 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
     HIPCHECK(hipEventRecord(b->ev1, b->stream));
     HIPCHECK(hipMemcpyAsync(out, b->d_out, sizeof(ps_fit_result) * njobs, hipMemcpyDeviceToHost, b->stream));
     HIPCHECK(hipStreamSynchronize(b->stream));
+    S.busy = false;
     float ms = 0;
     HIPCHECK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     b->kernel_ms += ms;
@@ -1638,7 +1727,7 @@ extern "C" int ps_batch_run(ps_batch *b, const double *conw_r, int njobs, const 
 }
 
 extern "C" int ps_test_batch_spread(const ps_batch *b) { return b->last_spread; }
-extern "C" void ps_test_batch_limits(ps_batch *b, size_t arena) { b->spread.limit = arena; }
+extern "C" void ps_test_batch_limits(ps_batch *b, size_t arena) { b->spread_limit = arena; }
 
 extern "C" int ps_batch_kernel_time(ps_batch *b, double *ms, int *launches, int reset) {
     if (!b) return ps_fail(PS_ERR_ARG, "ps_batch_kernel_time: null batch");
@@ -1682,6 +1771,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     if (rc != PS_OK) return rc;
     // few vectors: their passes spread over the chip
     bool spread = use_v2(h) && long(nvec) * h->P2.npass <= kSpreadPasses && spread_pays(h, nvec, true);
+    Spread S(h->device, h->stream, h->spread_limit);
     std::vector<psk::SpreadJob> sjobs;
     std::vector<psk::SpreadTask> stasks;
     if (spread) {
@@ -1690,10 +1780,8 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
             sjobs.back().part0 = v * h->P2.npass;
         }
         stasks = spread_tasks(sjobs, h->slots2);
-        auto layout = [&] {
-            return spread_layout(h->spread, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac);
-        };
-        spread = spread_reserve(h->spread, layout());
+        auto layout = [&] { return spread_layout(S, nvec, stasks.size(), size_t(nvec) * h->P2.npass, h->mfit, h->nfac); };
+        spread = S.reserve(layout());
         if (spread) layout();
     }
     h->last_spread = spread ? nvec : 0;
@@ -1718,7 +1806,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         return rc;
     HIPCHECK(hipMemcpyAsync(E.a, a, sizeof(double) * nv * h->ma, hipMemcpyHostToDevice, h->stream));
     if (spread) {
-        Spread &S = h->spread;
+        S.busy = true;
         HIPCHECK(hipMemcpyAsync(S.jobs, sjobs.data(), sizeof(sjobs[0]) * sjobs.size(), hipMemcpyHostToDevice, h->stream));
         HIPCHECK(hipMemcpyAsync(S.tasks, stasks.data(), sizeof(stasks[0]) * stasks.size(), hipMemcpyHostToDevice, h->stream));
     }
@@ -1732,7 +1820,6 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
             if (user[i]) at += size_t(n) * len[i];
         }
         if (spread) {
-            Spread &S = h->spread;
             auto launch = [&](auto *kern) {
                 hipLaunchKernelGGL(kern, dim3(stasks.size()), dim3(psk::kWG2), 0, h->stream, S.jobs, S.tasks, S.B, va, dev[3],
                                    dev[4]);
@@ -1840,6 +1927,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     for (hipError_t e : errs)
         if (e != hipSuccess) return ps_fail(PS_ERR_DEVICE, "ps_eval: copy failed: %s", hipGetErrorString(e));
     HIPCHECK(hipStreamSynchronize(h->stream));
+    S.busy = false;
     float ms = 0;
     HIPCHECK(hipEventElapsedTime(&ms, h->ev0, h->ev1));
     h->kernel_ms += ms;
@@ -1863,7 +1951,6 @@ extern "C" void ps_release(ps_handle *h) {
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     for (void *p : h->owned) hipFree(p);
-    hipFree(h->spread.arena);
     if (h->ev.pin) hipHostFree(h->ev.pin);
     if (h->ev.copy) hipStreamDestroy(h->ev.copy);
     for (auto *v : {&h->ev.chunk, &h->ev.slot})
@@ -1874,5 +1961,6 @@ extern "C" void ps_release(ps_handle *h) {
     if (h->ev0) hipEventDestroy(h->ev0);
     if (h->ev1) hipEventDestroy(h->ev1);
     if (h->stream) hipStreamDestroy(h->stream);
+    arenas().handles(h->device, -1);
     delete h;
 }

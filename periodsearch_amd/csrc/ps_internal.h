@@ -18,4 +18,6 @@ int ps_test_batch_spread(const ps_batch *b);
 // Caps what later calls can have: bytes of device memory for the spread form's buffers.
 void ps_test_limits(ps_handle *h, size_t arena);
 void ps_test_batch_limits(ps_batch *b, size_t arena);
+// The bytes of a device's idle arenas (the spread form's memory) and its open handles.
+size_t ps_test_arenas(int device, int *handles);
 }

@@ -1,6 +1,9 @@
 """Calls whose buffers cannot be had (the limits are forced on the handle or batch): they take the other form and
-return the same bits, as they did before there was a choice of forms."""
+return the same bits, as they did before there was a choice of forms; and the spread form's memory, which the
+handles of a device share."""
 import ctypes as C
+import gc
+import threading
 
 import numpy as np
 import pytest
@@ -81,3 +84,70 @@ def test_no_room_to_spread():
     finally:
         a.close()
         b.close()
+
+
+def arenas():
+    fn = lib().ps_test_arenas
+    fn.argtypes, fn.restype = [C.c_int, C.POINTER(C.c_int)], C.c_size_t
+    n = C.c_int()
+    return fn(0, C.byref(n)), n.value
+
+
+def test_open_handles_share_the_spread_memory():
+    """Handles that stay open after a spread call hold none of its memory; what waits for the next call is
+    bounded and goes with the last handle."""
+    gc.collect()
+    others = arenas()[1]
+    text = passes(6, 6, 20)
+    searches = [prepared(text) for _ in range(6)]
+    try:
+        conw = searches[0].info()["conw_r0"]
+        freq, pole = searches[0].freq(1 + np.arange(100) // 10), 1 + np.arange(100) % 10
+        want = None
+        for s in searches:
+            got = s.fit_batch(freq, pole, conw)
+            assert spread(s) == 100
+            want = got if want is None else want
+            same(got, want, "another handle's arena")
+        one = 100 * 20 * 24576  # the Gram blocks of one call
+        assert arenas()[1] == others + 6
+        if others == 0:
+            assert one <= arenas()[0] < 2 * one
+        assert arenas()[0] < 3 * (200 << 20)
+    finally:
+        for s in searches:
+            s.close()
+    assert arenas()[1] == others
+    if others == 0:
+        assert arenas()[0] == 0
+
+
+def test_threads_with_handles_of_their_own():
+    """Calls that overlap on streams of their own never share an arena."""
+    shapes = [passes(6, 6, 12), passes(3, 4, 20), passes(6, 8, 10), passes(4, 5, 16)]
+    searches = [prepared(t) for t in shapes]
+    try:
+        jobs = []
+        for s in searches:
+            n = 1 + np.arange(60)
+            jobs.append((s, s.freq(1 + n // 10), 1 + n % 10, s.info()["conw_r0"]))
+        want = [s.fit_batch(f, p, c) for s, f, p, c in jobs]
+        got = [[None] * 5 for _ in jobs]
+
+        def work(i):
+            s, f, p, c = jobs[i]
+            for r in range(5):
+                m = 60 - 10 * r  # arenas of several sizes
+                got[i][r] = s.fit_batch(f[:m], p[:m], c)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        for i, w in enumerate(want):
+            for r in range(5):
+                same(got[i][r], w[:60 - 10 * r], (i, r))
+    finally:
+        for s in searches:
+            s.close()
