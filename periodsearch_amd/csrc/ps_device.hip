@@ -443,7 +443,7 @@ struct ps_handle {
         hipStream_t copy = nullptr;  // outputs of a chunk leave while the next one is computed
         std::vector<hipEvent_t> chunk, slot;
     } ev;
-    size_t spread_limit = size_t(-1);  // of the spread form's memory (ps_test_limits)
+    size_t spread_limit = size_t(-1), pinned_limit = size_t(-1);  // of device and pinned memory (ps_test_limits)
     int last_spread = 0;  // fits or vectors of the last call that took the spread form
     std::vector<double> wq2_host;
     double *d_wq2 = nullptr;
@@ -1105,7 +1105,10 @@ int spread_rest(const ps_handle *h, int nfits) {
 
 extern "C" int ps_test_spread(const ps_handle *h) { return h->last_spread; }
 extern "C" size_t ps_test_arenas(int device, int *handles) { return arenas().idle_bytes(device, handles); }
-extern "C" void ps_test_limits(ps_handle *h, size_t arena) { h->spread_limit = arena; }
+extern "C" void ps_test_limits(ps_handle *h, size_t arena, size_t pinned) {
+    h->spread_limit = arena;
+    h->pinned_limit = pinned;
+}
 
 extern "C" int ps_set_precision(ps_handle *h, int precision) {
     if (!h) return ps_fail(PS_ERR_ARG, "ps_set_precision: null handle");
@@ -1873,12 +1876,27 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     if (!pieces.empty()) {
         if (E.cpin < threads * slot) {
             (void)hipHostFree(E.pin);
+            E.pin = nullptr;
             E.cpin = 0;
-            if (hipHostMalloc(&E.pin, threads * slot * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-                E.pin = nullptr;
-                return ps_fail(PS_ERR_NOMEM, "ps_eval: pinned staging allocation failed");
+            if (threads * slot * sizeof(double) <= h->pinned_limit &&
+                hipHostMalloc(&E.pin, threads * slot * sizeof(double), hipHostMallocDefault) == hipSuccess)
+                E.cpin = threads * slot;
+            else
+                (void)hipGetLastError();
+        }
+        if (!E.pin) {
+            // no pinned memory to be had: array by array, through the runtime's own staging
+            for (int c = 0; c < nchunk; ++c) {
+                const int v0 = c * step, n = std::min(step, nvec - v0);
+                const double *at = E.out + size_t(v0) * per;
+                for (int i = 0; i < 5; ++i) {
+                    if (!user[i]) continue;
+                    HIPCHECK(hipMemcpyAsync(user[i] + size_t(v0) * len[i], at, size_t(n) * len[i] * sizeof(double),
+                                            hipMemcpyDeviceToHost, h->stream));
+                    at += size_t(n) * len[i];
+                }
             }
-            E.cpin = threads * slot;
+            pieces.clear();
         }
         if (!E.copy && nchunk > 1) HIPCHECK(hipStreamCreateWithFlags(&E.copy, hipStreamNonBlocking));
         while (int(E.slot.size()) < threads) {

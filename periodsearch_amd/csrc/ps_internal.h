@@ -15,8 +15,9 @@ extern "C" {
 // The fits (ps_fit_batch, ps_scan, ps_batch_run) or vectors (ps_eval) of the last call that took the spread form.
 int ps_test_spread(const ps_handle *h);
 int ps_test_batch_spread(const ps_batch *b);
-// Caps what later calls can have: bytes of device memory for the spread form's buffers.
-void ps_test_limits(ps_handle *h, size_t arena);
+// Caps what later calls can have: bytes of device memory for the spread form's buffers, of pinned memory for
+// the outputs of ps_eval.
+void ps_test_limits(ps_handle *h, size_t arena, size_t pinned);
 void ps_test_batch_limits(ps_batch *b, size_t arena);
 // The bytes of a device's idle arenas (the spread form's memory) and its open handles.
 size_t ps_test_arenas(int device, int *handles);

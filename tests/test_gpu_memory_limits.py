@@ -14,10 +14,13 @@ from tests.test_gpu_spread_rule import passes, prepared, spread
 pytestmark = pytest.mark.gpu
 
 
-def limit(ps, *args):
+ALL = C.c_size_t(-1).value
+
+
+def limit(ps, arena=ALL, pinned=ALL):
     fn = lib().ps_test_limits
-    fn.argtypes, fn.restype = [C.c_void_p] + [C.c_size_t] * len(args), None
-    fn(ps._handle(), *args)
+    fn.argtypes, fn.restype = [C.c_void_p, C.c_size_t, C.c_size_t], None
+    fn(ps._handle(), arena, pinned)
 
 
 def batch_limit(b, arena):
@@ -81,6 +84,28 @@ def test_no_room_to_spread():
         assert (spread(a), spread(b)) == (9, 0)
         for k in want:
             assert np.array_equal(got[k], want[k]), k
+    finally:
+        a.close()
+        b.close()
+
+
+def test_evaluations_without_pinned_memory():
+    """Short lists and lists in chunks, all outputs and some of them."""
+    text = passes(3, 4, 2)
+    a, b = prepared(text), prepared(text)
+    try:
+        limit(b, pinned=0)
+        conw = a.info()["conw_r0"]
+        n = 2 * a.info()["slots"] + 3
+        vec = np.zeros((n, a.info()["ma"]))
+        nc = a.info()["ncoef"]
+        vec[:, :nc], vec[:, nc] = a.geometry()["cg_first"], np.linspace(0.5, 2.5, n)
+        vec[:, nc + 2] = 2 * np.pi * 24 * a.freq(1)
+        vec[:, nc + 3:] = 0.5, 0.1, -0.5, -2.0, 1.0
+        for m, raw in ((1, True), (9, False), (n, True), (n, False)):
+            want, got = a.eval(vec[:m], conw, raw=raw), b.eval(vec[:m], conw, raw=raw)
+            for k in want:
+                assert np.array_equal(got[k], want[k]), (m, k)
     finally:
         a.close()
         b.close()
