@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from periodsearch_amd import PS_KERNEL_JFREE, PeriodSearch
+from periodsearch_amd import _lib as L
 from tests import oracle_binding as ob
 from tests.test_gpu_orbits import problem
 
@@ -81,5 +82,48 @@ def test_any_lommel_seeliger_weight(cls, cl_free):
                 br, dy = orc.bright(a, arr["ee"][p], arr["ee0"][p], arr["tim"][p])
                 assert abs(got["ymod"][v, p] - br) <= 1e-13 * abs(br), p
                 assert np.abs(got["dyda"][v, p] - dy).max() <= 1e-12 * np.abs(dy).max(), p
+    finally:
+        ps.close()
+
+
+def call(ps, vecs, conw, keys):
+    """ps_eval with the named outputs only."""
+    info, n = ps.info(), len(vecs)
+    shape = {"alpha": (n, info["mfit"], info["mfit"]), "beta": (n, info["mfit"]), "chisq": (n,),
+             "ymod": (n, info["npts"]), "dyda": (n, info["npts"], info["ma"])}
+    out = {k: np.full(shape[k], np.nan) for k in keys}
+    ptr = [out[k].ctypes.data_as(L.DP) if k in out else None for k in KEYS]
+    L.check(L.lib().ps_eval(ps._handle(), n, vecs.ctypes.data_as(L.DP), float(conw), *ptr), "ps_eval")
+    return out
+
+
+@pytest.mark.parametrize("keys", [KEYS, KEYS[:3], ("alpha",), ("chisq", "ymod", "dyda"), ()], ids=str)
+def test_long_lists_match_short_calls(keys):
+    """Chunks of whole rounds and a remainder of one, of a few and of none; pieces that cross the arrays' ends."""
+    ps = prepared(3, 3, 5, 2, 30, 0)  # 12 KB of raw rows a vector
+    try:
+        conw, slots = ps.info()["conw_r0"], ps.info()["slots"]
+        vecs = vectors(ps, 2 * slots + 3)
+        parts = [ps.eval(vecs[i:i + 7], conw, raw=True) for i in range(0, len(vecs), 7)]
+        want = {k: np.concatenate([p[k] for p in parts]) for k in KEYS}
+        for n in (2 * slots + 3, 2 * slots, slots + 1):
+            got = call(ps, vecs[:n], conw, keys)
+            for k in keys:
+                assert np.array_equal(got[k], want[k][:n]), (n, k)
+    finally:
+        ps.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 7, 8, 9, 30])
+def test_results_of_one_to_several_pieces(n):
+    ps = prepared(6, 6, 4, 20, 50, 300)  # 0.6 MB of raw rows a vector: results of one piece to eighteen
+    try:
+        conw = ps.info()["conw_r0"]
+        vecs = vectors(ps, n)
+        got = call(ps, vecs, conw, KEYS)
+        for i in range(n):
+            one = call(ps, vecs[i:i + 1], conw, KEYS)
+            for k in KEYS:
+                assert np.array_equal(got[k][i], one[k][0]), (i, k)
     finally:
         ps.close()
