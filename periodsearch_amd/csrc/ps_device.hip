@@ -1862,8 +1862,8 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     // one thread at the runtime's hands moved 99 MB of normal equations in 9 ms, page faults of fresh arrays
     // included, after 7 ms of kernels; four move them while the kernels run.  One thread alone copies, waits
     // and moves on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
-    // to 400 points) takes 1123 us with one, 1043 with two, 1016 with four; 6.6 MB of raw rows 675, 571, 539.
-    // Smaller pieces cost more than they overlap (64 KiB instead of 1 MiB: 1.1 to 2 times the call).
+    // to 400 points) takes 1123 us with one, 1044 with two, 1016 with four; 6.6 MB of raw rows 647, 478, 472.
+    // Smaller pieces cost more than they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
     struct Piece {
         int chunk;
         size_t off, n;  // in doubles, within the device buffer
