@@ -17,8 +17,8 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -146,9 +146,10 @@ bool build_schedule(const std::vector<int> &lc_start, const std::vector<int> &lc
 }
 
 // The symmetry orbits of a geometry (ps_orbit.h): for every orbit the members' mean normal (they differ by
-// a few 1e-16, their own rounding) and the representative's harmonics, for every facet its entry (8 * orbit + 2k + (1: -n_k)).  Returns false where the mesh or the
-// coefficient set is not of that kind (a caller may fill ps_geometry itself); every member's normal and
-// harmonics are compared with what the symmetry gives, to a few units of rounding.
+// a few 1e-16, their own rounding) and the representative's harmonics, for every facet its entry
+// (8 * orbit + 2k + (1: -n_k)).  Returns false where the mesh or the coefficient set is not of that kind (a
+// caller may fill ps_geometry itself); every member's normal and harmonics are compared with what the
+// symmetry gives, to a few units of rounding.
 struct Orbits {
     int L = 0, n = 0;
     std::vector<double> table;
@@ -216,7 +217,10 @@ bool build_orbits(const ps_geometry &g, Orbits &ob) {
         const double dc = v(c.cos), ds = c.m ? v(c.sin) : 0.0, w = c.s ? ds * c4 + dc * s4 : dc * c4 - ds * s4;
         return sg && (c.l & 1) ? -w : w;
     };
-    constexpr double kNorTol = 1e-14, kHarmTol = 1e-13;
+    // The normals of an orbit are replaced by one and its turned copies, without a correction, so only the
+    // rounding of trifac.c's own meshes passes (up to 1.1e-15 at 8 rows).  The harmonics' differences, larger
+    // by the order of the polynomials, are put back by the correction rows to three digits.
+    constexpr double kNorTol = 2e-15, kHarmTol = 1e-13;
     int norb = 0;
     for (int r = 0; r < g.nfac; ++r) {
         const double *n = g.nor + 3 * r;
@@ -1938,9 +1942,10 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         errs[w] = e;
     };
     std::vector<std::thread> pool;
+    pool.reserve(threads);
     try {
         for (int w = 1; w < threads; ++w) pool.emplace_back(work, w);
-    } catch (const std::system_error &) {  // no thread to be had: its share runs here
+    } catch (const std::exception &) {  // no thread, or no memory for one: its share runs here
     }
     work(0);
     for (int w = 1 + int(pool.size()); w < threads; ++w) work(w);

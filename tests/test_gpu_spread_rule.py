@@ -110,3 +110,18 @@ def test_fits_of_no_iteration_evaluate_nothing():
                 assert (got[k] == 0).all(), (k, got[k])
     finally:
         ps.close()
+
+
+@pytest.mark.parametrize("off,expect", [(0.0, 10), (4e-15, 0)])
+def test_only_rounding_passes_for_symmetry(off, expect):
+    """A mesh whose normals are off the symmetry by more than rounding is not folded (by tiles nothing is spread)."""
+    ps = PeriodSearch.from_text(passes(6, 6, 10))
+    g = ps._geo.contents
+    np.ctypeslib.as_array(g.nor, (g.nfac * 3,))[0] += off
+    ps.prepare(device=0)
+    ps.set_kernel(PS_KERNEL_JFREE)
+    try:
+        ps.fit_batch(ps.freq(np.full(10, 2)), np.arange(1, 11), ps.info()["conw_r0"])
+        assert spread(ps) == expect
+    finally:
+        ps.close()
