@@ -1069,9 +1069,11 @@ int iteration_cap(const ps_handle *h) { return std::max({h->P.n_iter_max, h->P.n
 
 // Whether n fits (or, evals, single evaluations) of a problem are faster spread than in one workgroup each,
 // in us an iteration.  Both forms pay for the solve; a workgroup of its own walks all passes, two to a CU
-// 1.5 times as long; the spread form takes spread_time and its launches and trips through memory: 14 us
-// and what the solves' workgroups read, or, for evaluations, 33 us (the jobs' and tasks' upload included)
-// and the tables' making.  The time of a pass, a fit over 3 + 0.1 mfit + norb (0.2 + 0.003 N): measured 8.9
+// 1.5 times as long; the spread form takes spread_time and its launches and trips through memory: 11 us
+// and what the solves' workgroups read, or, for evaluations, 31 us (the jobs' and tasks' upload included)
+// and the tables' making.  Both constants and the margins are those that choose best at 200 lists of fits and
+// 168 of evaluations measured in both forms (1 to 40 passes, Lmax 2 to 6, lists of 1 to 281): the rule is
+// within 5 % of the faster form at every one, where the number of fits alone was off by up to 1.8 times.  The time of a pass, a fit over 3 + 0.1 mfit + norb (0.2 + 0.003 N): measured 8.9
 // (Lmax 2, 128 facets), 14.5 (3, 288), 13 (4, 200), 21 (6, 288), 30.5 (6, 512).
 // Measured on both sides of the rule, one workgroup each / spread, us for 6 iterations: Lmax 6, 288 facets,
 // 10 fits of 1 pass 484 / 590, 2 passes 632 / 586; 200 fits of 4 passes 934 / 994, 10 passes 1816 / 1637;
@@ -1089,9 +1091,9 @@ bool spread_pays(const ps_handle *h, int n, bool evals) {
         const std::vector<psk::SpreadJob> jobs(std::min(left, most), spread_job(h, 0, 0, 0, 0));
         const int q = spread_length(jobs, h->slots2);
         spread += pass * spread_time(jobs, q, h->slots2);
-        spread += evals ? 33 + 0.012 * jobs.size() * ((np + q - 1) / q) : 14 + 1.7e-5 * jobs.size() * h->mfit * h->mfit;
+        spread += evals ? 31 + 0.012 * jobs.size() * ((np + q - 1) / q) : 11 + 1.7e-5 * jobs.size() * h->mfit * h->mfit;
     }
-    return (evals ? 1.1 : 1.05) * spread < solo;
+    return (evals ? 1.1 : 1.03) * spread < solo;
 }
 
 // The fits of a list that are spread: those past whole rounds of the resident workgroups.  A piece of spread
