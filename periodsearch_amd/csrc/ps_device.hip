@@ -1863,11 +1863,13 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
             HIPCHECK(hipEventRecord(E.chunk[c], h->stream));
         }
     }
-    // Outputs to the caller's (pageable) arrays through pinned slots.  A result of more than a piece is copied by
+    // Outputs to the caller's (pageable) arrays through pinned slots.  A chunk of more than a piece is copied by
     // up to four threads, each with a slot of its own, a piece at a time, chunk by chunk as the kernels finish:
     // one thread at the runtime's hands moved 99 MB of normal equations in 9 ms, page faults of fresh arrays
-    // included, after 7 ms of kernels; four move them while the kernels run.  One thread alone copies, waits
-    // and moves on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
+    // included, after 7 ms of kernels; four move them while the kernels run.  Chunks of one piece leave while
+    // the next one is computed, and making threads costs more than they save (1500 vectors of 2.9 MB in six
+    // chunks: 1179 us with one thread, 1246 with four).  In larger ones a thread alone copies, waits and moves
+    // on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
     // to 400 points) takes 1123 us with one, 1044 with two, 1016 with four; 6.6 MB of raw rows 647, 478, 472.
     // Smaller pieces cost more than they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
     struct Piece {
@@ -1880,7 +1882,8 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         const size_t b0 = size_t(c) * step * per, b1 = std::min(nv, size_t(c + 1) * step) * per;
         for (size_t o = b0; o < b1; o += kPiece) pieces.push_back({c, o, std::min(kPiece, b1 - o)});
     }
-    const int threads = int(std::min<size_t>(4, std::max<size_t>(1, pieces.size())));
+    const size_t chunk_pieces = (std::min(nv, size_t(step)) * per + kPiece - 1) / kPiece;  // of the largest chunk
+    const int threads = int(std::min<size_t>(4, std::max<size_t>(1, chunk_pieces)));
     const size_t slot = std::min(kPiece, nv * per);
     if (!pieces.empty()) {
         if (E.cpin < threads * slot) {
