@@ -1806,9 +1806,14 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     double *const user[5] = {alpha, beta, chisq, ymod, dyda};
     size_t per = 0;
     for (int i = 0; i < 5; ++i) per += user[i] ? len[i] : 0;
-    // chunks of whole rounds of the resident workgroups, at most eight
+    // Chunks of whole rounds of the resident workgroups, at most eight, of at least 8 MiB of outputs: between two
+    // chunks the chip drains, and less than that is copied in the time this takes (1500 vectors of 2.9 MB, long
+    // lightcurves: 1204 us in one chunk, 1301 in six; 4000 of 32 MB 4297 in one, 4134 in four; 4096 of 100 MB 10046
+    // in one, 8931 in eight).
     const int slots = use_v2(h) ? h->slots2 : h->slots;
-    const int rounds = (nvec + slots - 1) / slots, step = spread ? nvec : slots * std::max(1, (rounds + 7) / 8);
+    const int rounds = (nvec + slots - 1) / slots;
+    const int most = int(std::min<size_t>(8, std::max<size_t>(1, nv * per * sizeof(double) >> 23)));
+    const int step = spread ? nvec : slots * ((rounds + most - 1) / most);
     const int nchunk = (nvec + step - 1) / step;
     auto &E = h->ev;
     if ((rc = grow(h, E.a, E.ca, nv * h->ma)) != PS_OK || (rc = grow(h, E.out, E.cout, nv * std::max<size_t>(per, 1))) != PS_OK)
@@ -1866,10 +1871,8 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     // Outputs to the caller's (pageable) arrays through pinned slots.  A chunk of more than a piece is copied by
     // up to four threads, each with a slot of its own, a piece at a time, chunk by chunk as the kernels finish:
     // one thread at the runtime's hands moved 99 MB of normal equations in 9 ms, page faults of fresh arrays
-    // included, after 7 ms of kernels; four move them while the kernels run.  Chunks of one piece leave while
-    // the next one is computed, and making threads costs more than they save (1500 vectors of 2.9 MB in six
-    // chunks: 1179 us with one thread, 1246 with four).  In larger ones a thread alone copies, waits and moves
-    // on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
+    // included, after 7 ms of kernels; four move them while the kernels run.  One thread alone copies, waits and
+    // moves on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
     // to 400 points) takes 1123 us with one, 1044 with two, 1016 with four; 6.6 MB of raw rows 647, 478, 472.
     // Smaller pieces cost more than they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
     struct Piece {

@@ -100,7 +100,7 @@ def call(ps, vecs, conw, keys):
 @pytest.mark.parametrize("keys", [KEYS, KEYS[:3], ("alpha",), ("chisq", "ymod", "dyda"), ()], ids=str)
 def test_long_lists_match_short_calls(keys):
     """Chunks of whole rounds and a remainder of one, of a few and of none; pieces that cross the arrays' ends."""
-    ps = prepared(3, 3, 5, 2, 30, 0)  # 12 KB of raw rows a vector
+    ps = prepared(5, 5, 5, 2, 30, 0)  # 36 KB of outputs a vector: up to three chunks
     try:
         conw, slots = ps.info()["conw_r0"], ps.info()["slots"]
         vecs = vectors(ps, 2 * slots + 3)
