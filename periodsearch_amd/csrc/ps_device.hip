@@ -1868,13 +1868,13 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
             HIPCHECK(hipEventRecord(E.chunk[c], h->stream));
         }
     }
-    // Outputs to the caller's (pageable) arrays through pinned slots.  A chunk of more than a piece is copied by
-    // up to four threads, each with a slot of its own, a piece at a time, chunk by chunk as the kernels finish:
-    // one thread at the runtime's hands moved 99 MB of normal equations in 9 ms, page faults of fresh arrays
-    // included, after 7 ms of kernels; four move them while the kernels run.  One thread alone copies, waits and
-    // moves on, piece by piece: the call of 200 vectors with 4.8 MB of normal equations (lightcurves of up
-    // to 400 points) takes 1123 us with one, 1044 with two, 1016 with four; 6.6 MB of raw rows 647, 478, 472.
-    // Smaller pieces cost more than they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
+    // Outputs to the caller's (pageable) arrays through pinned slots, a piece at a time, chunk by chunk as the
+    // kernels finish.  One thread alone copies, waits and moves on, so a chunk of more than a piece is shared by
+    // two threads with a slot each, and one of 8 MiB by four: 250 vectors with 6 MB of normal equations
+    // (lightcurves of up to 400 points) take 1246 us with one, 1117 with two, 1084 with four; 5.5 MB of raw rows
+    // 579, 446, 433; 4096 vectors of 100 MB 11.1, 7.3 and 6.6 ms.  Below 8 MiB more than two threads gain little
+    // and the first call of a handle, which makes their slots, loses up to 1 ms.  Smaller pieces cost more than
+    // they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
     struct Piece {
         int chunk;
         size_t off, n;  // in doubles, within the device buffer
@@ -1886,7 +1886,7 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         for (size_t o = b0; o < b1; o += kPiece) pieces.push_back({c, o, std::min(kPiece, b1 - o)});
     }
     const size_t chunk_pieces = (std::min(nv, size_t(step)) * per + kPiece - 1) / kPiece;  // of the largest chunk
-    const int threads = int(std::min<size_t>(4, std::max<size_t>(1, chunk_pieces)));
+    const int threads = chunk_pieces >= 8 ? 4 : chunk_pieces > 1 ? 2 : 1;
     const size_t slot = std::min(kPiece, nv * per);
     if (!pieces.empty()) {
         if (E.cpin < threads * slot) {
