@@ -442,8 +442,11 @@ struct ps_handle {
     struct EvalBuffers {  // ps_eval's staging, kept between calls
         double *a = nullptr, *out = nullptr;  // device: the vectors, the outputs chunk by chunk
         size_t ca = 0, cout = 0;
-        char *pin = nullptr;  // pinned: one slot per copying thread
-        size_t cpin = 0;
+        struct Slot {
+            double *p = nullptr;
+            size_t n = 0;
+        };
+        std::vector<Slot> pin;  // pinned: one slot per copying thread
         hipStream_t copy = nullptr;  // outputs of a chunk leave while the next one is computed
         std::vector<hipEvent_t> chunk, slot;
     } ev;
@@ -1870,11 +1873,12 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     }
     // Outputs to the caller's (pageable) arrays through pinned slots, a piece at a time, chunk by chunk as the
     // kernels finish.  One thread alone copies, waits and moves on, so a chunk of more than a piece is shared by
-    // two threads with a slot each, and one of 8 MiB by four: 250 vectors with 6 MB of normal equations
+    // two threads with a slot each, and one of 8 pieces by four: 250 vectors with 6 MB of normal equations
     // (lightcurves of up to 400 points) take 1246 us with one, 1117 with two, 1084 with four; 5.5 MB of raw rows
-    // 579, 446, 433; 4096 vectors of 100 MB 11.1, 7.3 and 6.6 ms.  Below 8 MiB more than two threads gain little
-    // and the first call of a handle, which makes their slots, loses up to 1 ms.  Smaller pieces cost more than
-    // they overlap (128 KiB instead of 1 MiB: 1.2 to 2.3 times the call).
+    // 579, 446, 433; 4096 vectors of 100 MB 11.1, 7.3 and 6.6 ms.  Below 8 MiB more than two threads gain little.
+    // A handle's first call, which allocates, has one there: a second one's slot costs 0.4 ms, and ending a
+    // thread while memory is being mapped took up to 5 ms.  Smaller pieces cost more than they overlap (512 KiB:
+    // 495 us for the 5.5 MB; 128 KiB: 1.2 to 2.3 times the call).
     struct Piece {
         int chunk;
         size_t off, n;  // in doubles, within the device buffer
@@ -1886,20 +1890,26 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
         for (size_t o = b0; o < b1; o += kPiece) pieces.push_back({c, o, std::min(kPiece, b1 - o)});
     }
     const size_t chunk_pieces = (std::min(nv, size_t(step)) * per + kPiece - 1) / kPiece;  // of the largest chunk
-    const int threads = chunk_pieces >= 8 ? 4 : chunk_pieces > 1 ? 2 : 1;
+    const int threads = chunk_pieces >= 8 ? 4 : chunk_pieces > 1 && !E.slot.empty() ? 2 : 1;
     const size_t slot = std::min(kPiece, nv * per);
+    bool pinned = true;
     if (!pieces.empty()) {
-        if (E.cpin < threads * slot) {
-            (void)hipHostFree(E.pin);
-            E.pin = nullptr;
-            E.cpin = 0;
+        if (int(E.pin.size()) < threads) E.pin.resize(threads);
+        for (int w = 0; w < threads; ++w) {
+            auto &p = E.pin[w];
+            if (p.n >= slot) continue;
+            (void)hipHostFree(p.p);
+            p = {};
             if (threads * slot * sizeof(double) <= h->pinned_limit &&
-                hipHostMalloc(&E.pin, threads * slot * sizeof(double), hipHostMallocDefault) == hipSuccess)
-                E.cpin = threads * slot;
-            else
+                hipHostMalloc(&p.p, slot * sizeof(double), hipHostMallocDefault) == hipSuccess) {
+                p.n = slot;
+            } else {
                 (void)hipGetLastError();
+                p = {};
+                pinned = false;
+            }
         }
-        if (!E.pin) {
+        if (!pinned) {
             // no pinned memory to be had: array by array, through the runtime's own staging
             for (int c = 0; c < nchunk; ++c) {
                 const int v0 = c * step, n = std::min(step, nvec - v0);
@@ -1924,8 +1934,9 @@ extern "C" int ps_eval(ps_handle *h, int nvec, const double *a, double conw_r, d
     std::mutex mu;  // the copy stream: a piece's wait, copy and event go together
     std::vector<hipError_t> errs(threads, hipSuccess);
     auto work = [&](int w) {
+        if (size_t(w) >= pieces.size()) return;
         hipError_t e = hipSetDevice(h->device);
-        double *buf = reinterpret_cast<double *>(E.pin) + w * slot;
+        double *buf = E.pin[w].p;
         for (size_t p = w; p < pieces.size() && e == hipSuccess; p += threads) {
             const Piece &pc = pieces[p];
             {
@@ -1985,7 +1996,7 @@ extern "C" void ps_release(ps_handle *h) {
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     for (void *p : h->owned) hipFree(p);
-    if (h->ev.pin) hipHostFree(h->ev.pin);
+    for (const auto &p : h->ev.pin) hipHostFree(p.p);
     if (h->ev.copy) hipStreamDestroy(h->ev.copy);
     for (auto *v : {&h->ev.chunk, &h->ev.slot})
         for (hipEvent_t e : *v) hipEventDestroy(e);
