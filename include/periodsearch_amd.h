@@ -139,6 +139,8 @@ void ps_geometry_free(ps_geometry *geo);
    Returns PS_ERR_UNSUPPORTED when mfit > 63, ma > 63 or nfac > 512 (Lmax <= 6 and nrows <= 8 are
    supported; the reference allows up to MAX_N_PAR = 200 parameters and MAX_N_FAC = 1000 facets). */
 int ps_prepare(const ps_input *in, const ps_geometry *geo, int device, ps_handle **out);
+/* PS_FP64 (the default) or PS_MIXED.  Mixed precision is the less exact option and, on meshes with symmetry
+   orbits (every mesh of ps_geometry_build up to degree 6), the slower one too: 0.6 to 0.7 times the FP64 speed. */
 int ps_set_precision(ps_handle *h, int precision);
 /* Sets the kernel form of single-problem FP64 fits (PS_KERNEL_*); batches and ps_fit_batch_noalloc always
    run the J-free form.  No counterpart in the reference (one CPU build). */
@@ -149,7 +151,8 @@ int ps_get_kernel(const ps_handle *h);
    x 10 poles at convexity weight conw_r, 2 x the J-free form's resident workgroups, the second of two
    launches of each form), sets the faster one and reports it in *kernel and the two times per fit
    (legacy, J-free) in ms_per_fit[2] (either may be NULL).  Results are kept per problem shape (ncoef,
-   nfac, npts, mfit, Lambert column, iteration cap) for the life of the process.  Mixed precision and
+   nfac, npts, mfit, Lambert column, iteration cap, symmetry orbits of the mesh, passes) for the life of the
+   process.  Mixed precision and
    problems the J-free form does not accept get PS_KERNEL_LEGACY without timing. */
 int ps_autotune(ps_handle *h, double conw_r, int *kernel, double *ms_per_fit);
 int ps_get_info(const ps_handle *h, ps_info *info);
@@ -184,9 +187,9 @@ int ps_fit_batch_noalloc(ps_handle *h, int nfits, const double *freq, const int 
    PS_ERR_ARG (precisions differ).  The handles must outlive the batch.
    ps_batch_run: njobs fits (job j: problem prob[j], frequency freq[j] in 1/h, pole pole[j] in 1..10, at
    convexity weight conw_r[prob[j]]) as one graph launch: a queue reset, then persistent workgroups
-   that claim jobs from a device work queue, longest first, until it is empty.  FP64 batches with little
-   work for the chip, or with a fit that outlasts the rest, run as two launches per iteration over the
-   passes of all fits instead.  out[j] equals ps_fit_batch's result for the same fit.  The graph is
+   that claim jobs from a device work queue, longest first, until it is empty.  FP64 fits with symmetry orbits that
+   are little work for the chip, or one of which outlasts the rest, run as two launches per iteration over
+   the passes of all of them instead.  out[j] equals ps_fit_batch's result for the same fit.  The graph is
    kept and replayed while the job counts repeat.
    ps_batch_kernel_time: device time of the batch's launches since the last reset (HIP events). */
 typedef struct ps_batch ps_batch;

@@ -153,7 +153,8 @@ bool build_schedule(const std::vector<int> &lc_start, const std::vector<int> &lc
 struct Orbits {
     int L = 0, n = 0;
     std::vector<double> table;
-    std::vector<unsigned> corr;  // [32 positions][orbit, one more][position][member]: member - symmetric, bfloat16 pairs
+    // member - symmetric, bfloat16 pairs: [32 positions][orbit, one more][position][member]
+    std::vector<unsigned> corr;
     std::vector<int> pos, coef;
 };
 unsigned bf16_bits(double x) {  // round to nearest even (finite x)
@@ -1076,13 +1077,15 @@ int iteration_cap(const ps_handle *h) { return std::max({h->P.n_iter_max, h->P.n
 // and what the solves' workgroups read, or, for evaluations, 31 us (the jobs' and tasks' upload included)
 // and the tables' making.  Both constants and the margins are those that choose best at 200 lists of fits and
 // 168 of evaluations measured in both forms (1 to 40 passes, Lmax 2 to 6, lists of 1 to 281): the rule is
-// within 5 % of the faster form at every one, where the number of fits alone was off by up to 1.8 times.  The time of a pass, a fit over 3 + 0.1 mfit + norb (0.2 + 0.003 N): measured 8.9
-// (Lmax 2, 128 facets), 14.5 (3, 288), 13 (4, 200), 21 (6, 288), 30.5 (6, 512).
+// within 5 % of the faster form at every one, where the number of fits alone was off by up to 1.8 times.
+// The time of a pass is a fit too, 3 + 0.1 mfit + norb (0.2 + 0.003 N): measured 8.9 (Lmax 2, 128 facets),
+// 14.5 (3, 288), 13 (4, 200), 21 (6, 288), 30.5 (6, 512).
 // Measured on both sides of the rule, one workgroup each / spread, us for 6 iterations: Lmax 6, 288 facets,
 // 10 fits of 1 pass 484 / 590, 2 passes 632 / 586; 200 fits of 4 passes 934 / 994, 10 passes 1816 / 1637;
 // 281 fits of 4 passes 1203 / 1540, 10 passes 2496 / 2212; Lmax 2, 128 facets, 10 fits of 2 passes 263 / 294,
 // 3 passes 325 / 284; one evaluation at Lmax 3, 288 facets, of 2 passes 75 / 97, 6 passes 132 / 91.
-// From 0.55 of the resident workgroups on, the tasks take too many rounds (figures: ps_spread.h).
+// Past 0.55 of the resident workgroups fits of many passes still gain (300 fits of 20: 1.3 times), fits of few lose
+// (300 of 5: 0.98, 384: 0.85); nothing is spread there (more figures: ps_spread.h).
 constexpr double kSpreadShare = 0.55;
 bool spread_pays(const ps_handle *h, int n, bool evals) {
     const int np = h->P2.npass;

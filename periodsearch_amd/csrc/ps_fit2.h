@@ -938,8 +938,8 @@ __device__ __forceinline__ double mrqcof2(const DevProblem &P, Shared2<NFM> &sh,
 }
 
 // ---------------------------------------------------------------------------------------------
-// The systems cholesky_solve declines: full-pivot Gauss-Jordan (gauss_errc.c:9-73) on sh.u.g.cov with right-hand side sh.da, four waves each
-// holding rows w, w + 4, ... in registers.  Returns 0, 1 (no valid pivot) or 2 (zero pivot); only the
+// The systems cholesky_solve declines: full-pivot Gauss-Jordan (gauss_errc.c:9-73) on sh.u.g.cov with
+// right-hand side sh.da, four waves each holding rows w, w + 4, ... in registers.  Returns 0, 1 (no valid pivot) or 2 (zero pivot); only the
 // solution is written back.
 //
 // The reference swaps the pivot row into row icol (:38-42).  Here rows stay in place and carry a label,

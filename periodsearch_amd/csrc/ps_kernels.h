@@ -85,7 +85,7 @@ struct DevProblem {
     const double *qsl; // [nsched] sig*Lpoints of a relative lightcurve's point (mrqcof.c:94), else 0
     // Symmetry orbits of the facets (ps_orbit.h; norb = 0: the mesh has none).  orb: a row per orbit and
     // one more; opos[f]: facet f's entry in the kernels' area table, 8 * orbit + 2k + (1: -n_k);
-    // scol / scoef: the row column / coefficient of each stream position; xcol: eight row columns
+    // scol / scoef: the row column / coefficient of each stream position; xcol: seven row columns
     // that hold no shape coefficient and not the residual.
     int norb;
     const double *orb;
@@ -252,6 +252,8 @@ __device__ inline void blmatrix_lds(double bet, double lam, SH &sh) {
         double bl[3][3], dbl[2][3][3];
         blmatrix(bet, lam, bl, dbl);
         for (int i = 0; i < 9; ++i) sh.bl[i] = bl[i / 3][i % 3];
+        // nothing reads dbl; without the store the materialised-Jacobian form, which alone declares it, is 1 %
+        // slower (its register allocation changes)
         if constexpr (requires { sh.dbl; })
             for (int i = 0; i < 18; ++i) sh.dbl[i] = dbl[i / 9][(i / 3) % 3][i % 3];
         for (int j = 0; j < 2; ++j)
@@ -1001,9 +1003,10 @@ __device__ inline double read_lane(double x, int l) {  // x of lane l (l wave-un
 // ever find diagonal elements).  Panels of 16 columns: the blocks left of the panel are subtracted on
 // v_mfma_f64_16x16x4f64, then lane i carries row i through the panel's columns in registers, the pivot
 // row's entries as scalars from v_readlane; row n becomes D^-1 L^-1 b on the way.  Back substitution
-// leaves x_k in lane k.  Returns false, with nothing decided, when a pivot is not a normal positive number
-// (not positive definite to rounding, a column of rounding noise or overflow, NaN): the caller then runs
-// gauss_errc's elimination, which has the reference's answer to such systems.
+// leaves x_k in lane k.  Returns false, with nothing decided, when a pivot is outside 1e-270 .. 1e270: zero or
+// negative (not positive definite to rounding), a denormal or overflowing column, NaN.  The caller then runs
+// gauss_errc's elimination, which has the reference's answer to such systems.  The test is absolute: a pivot
+// that is rounding noise beside its diagonal but positive passes, as it does in the elimination.
 //
 // What bounds it: the chain of one column (read a lane, reciprocal, scale, update: about 100 cycles), 55
 // times.  The elimination it stands for takes 55 workgroup barriers and a pivot search over the whole

@@ -20,11 +20,15 @@
 // issue slots, so the VALU form loses nothing.)  A pass of 128 rows is two groups of 64 points; the two
 // waves of a group take alternate halves of the orbits and add their sums through the pass's LDS rows.
 //
-// What bounds it: FP64 issue.  Per orbit and 64 points 215 VALU instructions and 4 v_rcp_f64 replace the
-// 8 x 2 x (73 VALU + 6 MFMA of 64 cycles) / 4 of the tile form (ps_fit2.h model_rows2): about 910 cycles
-// instead of 2700, plus about 190 for the correction.  Measured, 2560 fits of 50 iterations: 2400 points and
-// 288 facets 352 -> 207 ms, 5000 points and 512 facets 1006 -> 505 ms; error of a Jacobian column against
-// extended precision 3.8e-16 and 3.2e-16 rms of its largest entry (tile form 4.0e-16, 3.7e-16).
+// What bounds it: FP64 issue.  Per orbit and 64 points 230 VALU instructions, 4 of them v_rcp_f64, replace the
+// 8 x 2 x (73 VALU + 6 MFMA of 64 cycles) / 4 of the tile form (ps_fit2.h model_rows2): 920 cycles of issue
+// instead of 2700.  Beside the other workgroup's wave on its SIMD a wave takes about 1650 cycles for them and
+// 370 for the correction (42 % and 10 % of its time at 2400 points and 288 facets, 58 % and 13 % at 5000 and
+// 512).  Measured when the form was made, 2560 fits of 50
+// iterations: 2400 points and 288 facets 352 -> 207 ms, 5000 points and 512 facets 1006 -> 505 ms; with the
+// steps since 178 and 484 ms (of these 189 -> 178 and 516 -> 484 by X's buffers on 16 bytes instead of 8
+// past them).  Error of a Jacobian column against extended precision 3.8e-16 and 3.2e-16 rms of its largest
+// entry (tile form 4.0e-16, 3.7e-16).
 #pragma once
 
 namespace psk {

@@ -13,12 +13,12 @@
 // Launches on one stream order the two; no workgroup waits for another inside a kernel.  The fit's state
 // lives in memory between them.  A finished fit's tasks and step return at once.
 //
-// What bounds it: the latency of one task, of the sum and solve, and two launches per iteration.  Measured,
-// 6 iterations, 2400 points, 288 facets: 10 fits 4.48 ms in one workgroup each, 1.16 ms spread; 100 fits
-// 4.51 and 2.11 ms; 530 fits of a smaller shape (18 past a full round) 14.0 and 9.6 ms; a batch of 240 fits
-// of 12 uneven problems 12.3 ms from the queue, 4.0 ms spread.  Against it: from 0.55 of the 512 resident
-// workgroups on, one workgroup each is no slower (5.9 ms for a full round at that shape; spread, 256 fits
-// 3.8 ms, 300 fits 4.7, 384 fits 5.6; at 600 points and Lmax 3 1.2 ms, spread 0.93, 1.23 and 1.45).
+// What bounds it: the latency of one task, of the sum and solve, and two launches per iteration (10 fits of 20
+// passes: 50 + 29 us of kernels in 92 us an iteration; 100 fits 185 + 32).  Measured, 6 iterations, one
+// workgroup each / spread: Lmax 6, 288 facets, 20 passes: 10 fits 3.27 / 0.63 ms, 100 fits 3.29 / 1.53, 256
+// fits 3.31 / 2.92, 300 fits 4.68 / 3.59, 384 fits 4.71 / 4.37, 448 fits 4.72 / 5.53; Lmax 3, 288 facets, 5
+// passes: 10 fits 0.71 / 0.39, 100 fits 0.72 / 0.46, 256 fits 0.72 / 0.64, 300 fits 0.92 / 0.94.  Fewer
+// passes: spread_pays in ps_device.hip, which chooses.
 #pragma once
 
 #include "ps_fit2.h"
